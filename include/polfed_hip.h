@@ -203,7 +203,8 @@ enum {
   PF_TUNE_WIDE = 6,
   PF_TUNE_GRAIN_SHUFFLE = 7,
   PF_TUNE_OCCUPANCY = 8,
-  PF_TUNE_ROW_PARTITION = 9
+  PF_TUNE_ROW_PARTITION = 9,
+  PF_TUNE_TEAM = 10
 };
 
 /* Force a launch knob of the row-interleaved step kernels for this operator:
@@ -221,6 +222,11 @@ enum {
  * that the row range each XCD owns gathers mostly its own rows; inputs and
  * outputs stay in the reference order and filter results are bit-identical;
  * the autotuner tries both orders),
+ * PF_TUNE_TEAM (-1 default; spin chains: 0 = one launch per filter step, 1, 2,
+ * 4, 8, 16 or 32 = the whole filter in one launch with this many blocks per
+ * column; ignored where the chain has no tables for it; the default rule and
+ * the autotuner choose, and any other forced knob selects the per-step
+ * launches, whose knobs they are),
  * PF_TUNE_RESET (drop forced and autotuned settings).  No reference
  * counterpart: launch tuning of this library. */
 int pf_op_set_tuning(pf_op* op, int32_t key, int32_t value);

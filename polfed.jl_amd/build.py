@@ -5,14 +5,16 @@ so that it travels with the source tree; nothing is installed elsewhere.
 """
 from __future__ import annotations
 
+import concurrent.futures
 import os
 import pathlib
 import subprocess
+import tempfile
 
 PKG = pathlib.Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OUT = PKG / "lib" / "libpolfed_hip.so"
-SOURCES = ["ops.hip", "dense.hip", "batch.hip", "packed.hip", "capi.cpp"]
+SOURCES = ["ops.hip", "team.hip", "batch.hip", "packed.hip", "dense.hip", "capi.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 FLAGS = [
@@ -20,17 +22,12 @@ FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     # packed FP32 instructions are kept out of every kernel of this library
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
 
-def build_library(verbose: bool = False) -> pathlib.Path:
-    """Compile every HIP source into lib/libpolfed_hip.so (always rebuilds)."""
-    OUT.parent.mkdir(parents=True, exist_ok=True)
-    tmp = OUT.with_suffix(".so.tmp")
-    cmd = [HIPCC, *FLAGS, "-o", str(tmp), *[str(CSRC / s) for s in SOURCES]]
+def _run(cmd, verbose: bool) -> None:
     res = subprocess.run(cmd, capture_output=True, text=True)
     if verbose or res.returncode != 0:
         msg = "\n".join(l for l in (res.stdout + res.stderr).splitlines()
@@ -39,6 +36,18 @@ def build_library(verbose: bool = False) -> pathlib.Path:
             print(msg)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed ({res.returncode}): {' '.join(cmd)}")
+
+
+def build_library(verbose: bool = False) -> pathlib.Path:
+    """Compile every HIP source into lib/libpolfed_hip.so (always rebuilds)."""
+    OUT.parent.mkdir(parents=True, exist_ok=True)
+    tmp = OUT.with_suffix(".so.tmp")
+    with tempfile.TemporaryDirectory() as d:  # the sources compile side by side
+        objs = [str(pathlib.Path(d) / (s + ".o")) for s in SOURCES]
+        cmds = [[HIPCC, *FLAGS, "-c", "-o", o, str(CSRC / s)] for s, o in zip(SOURCES, objs)]
+        with concurrent.futures.ThreadPoolExecutor(os.cpu_count() or 1) as pool:
+            list(pool.map(lambda c: _run(c, verbose), cmds))
+        _run([HIPCC, *FLAGS, "-shared", "-o", str(tmp), *objs], verbose)
     os.replace(tmp, OUT)
     return OUT
 

@@ -967,6 +967,7 @@ extern "C" int pf_op_create_spin_chain(pf_handle* h, int32_t L, int32_t Lup, int
                            op->pstates, (int64_t)D, L, nbonds, dfields, dbi, dbj, djd, op->pdiag);
         PF_HIP(hipGetLastError());
       }
+      op->team = P.tsplit > 0 ? team_build(P, C.data(), states.data(), op->diag) : nullptr;
       PF_HIP(hipDeviceSynchronize());
       (void)hipFree(dfields);
       (void)hipFree(dbi);
@@ -1056,6 +1057,7 @@ extern "C" int pf_op_destroy(pf_op* op) {
   if (op->prow) (void)hipFree(op->prow);
   if (op->pent) (void)hipFree(op->pent);
   if (op->pvals) (void)hipFree(op->pvals);
+  team_destroy(op->team);
   op->fbuf.release();
   op->kpart.release();
   delete op;
@@ -1218,6 +1220,13 @@ static void filter_body(pf_op* op, int32_t dtype, int32_t polytype, const double
   double phi0, phi1, a_tmp, b_tmp;
   poly_phi(polytype, phi0, phi1);
   poly_props(polytype, 1, a_tmp, b_tmp);
+  if (const int T = team_plan(op, dtype, polytype, order, X, ldx, Y, ldy, ncols)) {
+    int nslots;
+    size_t slot;
+    void* w = work(team_work_bytes(op, dtype, order, ncols, T, &nslots, &slot));
+    team_filter(op, dtype, polytype, coeffs, order, X, ldx, Y, ldy, ncols, T, w, st);
+    return;
+  }
   const Affine af = op->affine(true);
   const size_t esz = dtype == PF_F64 ? 8 : 4;
   const int cmax = chunk_cols(dtype);
@@ -1436,6 +1445,11 @@ extern "C" int pf_op_set_tuning(pf_op* op, int32_t key, int32_t value) {
     } else if (key == PF_TUNE_ROW_PARTITION) {
       PF_REQUIRE(value >= -1 && value <= 1, "tuning: row partition is -1, 0 or 1");
       op->force.part = value;
+    } else if (key == PF_TUNE_TEAM) {
+      PF_REQUIRE(value == -1 || value == 0 || value == 1 || value == 2 || value == 4 ||
+                     value == 8 || value == 16 || value == 32,
+                 "tuning: blocks per column -1, 0, 1, 2, 4, 8, 16 or 32");
+      op->force.team = value;
     } else if (key == PF_TUNE_RESET) {
       op->force = TuneCfg{};
       op->tuned.clear();
@@ -1537,6 +1551,37 @@ extern "C" int pf_autotune(pf_op* op, int32_t dtype, int32_t ncols, int32_t nste
       if (cd.us < 0.99 * best) {
         best = cd.us;
         bestc = cd.c;
+      }
+    }
+    // the one-launch filter against the best of them: a filter of this many
+    // steps (on zeros, as above), its begin and end launches included
+    double team_us = 1e300;
+    bestc.team = 0;
+    if (const int T = team_best(op, dtype, ncols, &team_us)) {
+      const int order = std::max(nsteps, 32);
+      int nslots;
+      size_t slot;
+      const size_t io = ((size_t)op->D * ncols * 8 + 255) & ~(size_t)255;
+      char* w = reinterpret_cast<char*>(
+          op->fbuf.get(2 * io + team_work_bytes(op, dtype, order, ncols, T, &nslots, &slot)));
+      PF_HIP(hipMemsetAsync(w, 0, 2 * io, st));
+      const std::vector<double> c(order + 1, 0.5);
+      double* X = reinterpret_cast<double*>(w);
+      double* Y = reinterpret_cast<double*>(w + io);
+      team_us = 1e300;
+      for (int round = 0; round < 3; ++round) {
+        PF_HIP(hipEventRecord(e0, st));
+        team_filter(op, dtype, PF_CHEBYSHEV, c.data(), order, X, op->D, Y, op->D, ncols, T, w + 2 * io,
+                    st);
+        PF_HIP(hipEventRecord(e1, st));
+        PF_HIP(hipEventSynchronize(e1));
+        float ms = 0.f;
+        PF_HIP(hipEventElapsedTime(&ms, e0, e1));
+        team_us = std::min(team_us, 1e3 * ms / order);
+      }
+      if (team_us < best) {
+        bestc.team = T;
+        best = team_us;
       }
     }
     (void)hipEventDestroy(e0);

@@ -158,7 +158,10 @@ struct TuneCfg {
   int shfl = -1;  // Quantum-Sun grain shuffles (-1 = default)
   int occ = -1;   // spin-chain 8-waves-per-SIMD variant (-1 = default)
   int part = -1;  // XCD partition row order in the drivers (-1 = default)
+  int team = -1;  // blocks per column of the team filter, 0: per-step launches (-1 = default)
 };
+
+struct TeamTables;  // team.hip
 
 }  // namespace pf
 
@@ -199,6 +202,7 @@ struct pf_op {
   double* pdiag = nullptr;      // diagonal in partition order
   void* prtab = nullptr;        // TA, then TB of the partition order
   uint32_t* pperm = nullptr;    // partition row -> reference rank
+  pf::TeamTables* team = nullptr;  // spin chain: tables of the one-launch filter (null: not eligible)
   pf::DevBuf fbuf;             // filter / KPM row-interleaved work blocks
   pf::TuneCfg force;           // pf_op_set_tuning overrides
   std::map<std::pair<int, int>, pf::TuneCfg> tuned;  // autotuned (dtype, s) configs
@@ -236,6 +240,21 @@ void launch_packed(pf_op* op, int dtype, int flags, const Layout& lay, int ncols
                    double cx, double ch, double cb, const void* X, const void* B2, const void* B3,
                    void* out, int64_t out_ld, hipStream_t st, double* dot_part, const void* P,
                    int dot_blocks);
+
+// The one-launch filter of spin chains (team.hip).  team_build: its tables, or
+// null when the chain does not fit; team_plan: blocks per column for a call, or
+// 0 for the per-step launches; team_best: the rule's choice and its time; team_work_bytes: device memory of a call.
+TeamTables* team_build(const ChainParams& ref, const uint32_t* C, const uint32_t* states,
+                       const double* diag_dev);
+void team_destroy(TeamTables* t);
+int team_plan(const pf_op* op, int dtype, int polytype, int order, const double* X, int64_t ldx,
+              const double* Y, int64_t ldy, int ncols);
+int team_best(const pf_op* op, int dtype, int ncols, double* us);
+size_t team_work_bytes(const pf_op* op, int dtype, int order, int ncols, int T, int* nslots,
+                       size_t* slot);
+void team_filter(pf_op* op, int dtype, int polytype, const double* coeffs, int order,
+                 const double* X, int64_t ldx, double* Y, int64_t ldy, int ncols, int T,
+                 void* work, hipStream_t st);
 
 // Looks up this device's address of pf_filter_noalloc's scratch array once per
 // device (ops.hip); called by pf_create with the device current.
