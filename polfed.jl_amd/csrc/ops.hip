@@ -1221,9 +1221,7 @@ static void filter_body(pf_op* op, int32_t dtype, int32_t polytype, const double
   poly_phi(polytype, phi0, phi1);
   poly_props(polytype, 1, a_tmp, b_tmp);
   if (const int T = team_plan(op, dtype, polytype, order, X, ldx, Y, ldy, ncols)) {
-    int nslots;
-    size_t slot;
-    void* w = work(team_work_bytes(op, dtype, order, ncols, T, &nslots, &slot));
+    void* w = work(team_work_bytes(op, dtype, order, ncols, T));
     team_filter(op, dtype, polytype, coeffs, order, X, ldx, Y, ldy, ncols, T, w, st);
     return;
   }
@@ -1370,7 +1368,19 @@ extern "C" int pf_kpm_moments(pf_op* op, int32_t dtype, int32_t N, int32_t R, co
     double* cscale = npart + (size_t)cmax * nb_norm;
     double* mu_dev = cscale + cmax;
     PF_HIP(hipMemsetAsync(mu_dev, 0, N * sizeof(double), st));
-    for (int c0 = 0; c0 < R; c0 += cmax) {
+    // one launch for a whole chunk of probes and all moments (team.hip): chunks of
+    // the columns whose norms the partials above hold
+    const int T = team_kpm_plan(op, dtype, N, std::min(R, cmax));
+    for (int c0 = 0; T && c0 < R; c0 += cmax) {
+      const int s = std::min(cmax, R - c0);
+      const double* src = probes + (int64_t)c0 * ldp;
+      hipLaunchKernelGGL(colnorm2_kernel, dim3(nb_norm, s), dim3(256), 0, st, src, ldp, op->D, npart);
+      hipLaunchKernelGGL(inv_sqrt_sum_kernel, dim3(1), dim3(64), 0, st, npart, nb_norm, s, cscale);
+      PF_HIP(hipGetLastError());
+      team_kpm(op, dtype, N, src, ldp, s, cscale, mu_dev, T,
+               op->fbuf.get(team_kpm_bytes(op, dtype, N, s, T)), st);
+    }
+    for (int c0 = 0; !T && c0 < R; c0 += cmax) {
       const int s = std::min(cmax, R - c0);
       const Layout lay = tuned_layout(op, dtype, s);
       const size_t blk = (size_t)op->D * s * esz;
@@ -1559,11 +1569,9 @@ extern "C" int pf_autotune(pf_op* op, int32_t dtype, int32_t ncols, int32_t nste
     bestc.team = 0;
     if (const int T = team_best(op, dtype, ncols, &team_us)) {
       const int order = std::max(nsteps, 32);
-      int nslots;
-      size_t slot;
       const size_t io = ((size_t)op->D * ncols * 8 + 255) & ~(size_t)255;
       char* w = reinterpret_cast<char*>(
-          op->fbuf.get(2 * io + team_work_bytes(op, dtype, order, ncols, T, &nslots, &slot)));
+          op->fbuf.get(2 * io + team_work_bytes(op, dtype, order, ncols, T)));
       PF_HIP(hipMemsetAsync(w, 0, 2 * io, st));
       const std::vector<double> c(order + 1, 0.5);
       double* X = reinterpret_cast<double*>(w);

@@ -250,11 +250,16 @@ void team_destroy(TeamTables* t);
 int team_plan(const pf_op* op, int dtype, int polytype, int order, const double* X, int64_t ldx,
               const double* Y, int64_t ldy, int ncols);
 int team_best(const pf_op* op, int dtype, int ncols, double* us);
-size_t team_work_bytes(const pf_op* op, int dtype, int order, int ncols, int T, int* nslots,
-                       size_t* slot);
+size_t team_work_bytes(const pf_op* op, int dtype, int order, int ncols, int T);
 void team_filter(pf_op* op, int dtype, int polytype, const double* coeffs, int order,
                  const double* X, int64_t ldx, double* Y, int64_t ldy, int ncols, int T,
                  void* work, hipStream_t st);
+// The KPM recurrence on the same kernels: mu[n] += sum over the columns (scaled by
+// colscale) of <x|T_n|x>, n < N.
+int team_kpm_plan(const pf_op* op, int dtype, int N, int ncols);
+size_t team_kpm_bytes(const pf_op* op, int dtype, int N, int ncols, int T);
+void team_kpm(pf_op* op, int dtype, int N, const double* X, int64_t ldx, int ncols,
+              const double* colscale, double* mu, int T, void* work, hipStream_t st);
 
 // Looks up this device's address of pf_filter_noalloc's scratch array once per
 // device (ops.hip); called by pf_create with the device current.

@@ -109,6 +109,9 @@ struct TeamArgs {
   uint32_t tab_lds, rows_lds;  // ends of the class tables and of the form's area in LDS
   TeamCtl* ctl;
   const double* coefs;
+  // KPM moments: 1/norm of each column, and the dots [step][2][column][kTeamUnits]
+  const double* colscale;
+  double* dots;
 };
 
 // Rows of the class tables: 2^kTeamLow strings or a whole small sector, each
@@ -322,10 +325,10 @@ __device__ __forceinline__ void outer_sum(BondSum<T, UNI>& s, const TeamArgs& A,
 // A lane's two rows of the caller's column (row + 1 only if `two`, else 0).
 template <typename T>
 __device__ __forceinline__ pair_t<T> x_pair(const TeamArgs& A, const double* X, int64_t row,
-                                            bool two) {
+                                            bool two, double f = 1.0) {
   pair_t<T> v;
-  v[0] = (T)X[A.perm ? A.perm[row] : row];
-  v[1] = two ? (T)X[A.perm ? A.perm[row + 1] : row + 1] : (T)0;
+  v[0] = (T)(X[A.perm ? A.perm[row] : row] * f);
+  v[1] = two ? (T)(X[A.perm ? A.perm[row + 1] : row + 1] * f) : (T)0;
   return v;
 }
 template <typename T>
@@ -349,8 +352,12 @@ struct TeamCoef {
 };
 // Factors of step k: out = cx X + ch H~ b2 + cb b3 (ch carries the scale of the
 // off-diagonal sum separately).
-template <typename T>
-__device__ __forceinline__ TeamCoef<T> team_coef(const TeamArgs& A, int k) {
+// The KPM recurrence T_j = 2 H~ T_{j-1} - T_{j-2} (T_1 = H~ T_0) takes the same
+// steps with no X term.
+template <typename T, bool KPM>
+__device__ __forceinline__ TeamCoef<T> team_coef(const TeamArgs& A, int j) {
+  if constexpr (KPM) return {(T)0, j == 1 ? (T)1 : (T)2, j == 1 ? (T)0 : (T)-1};
+  const int k = A.order - j;
   double alpha, beta, dummy;
   const double ck = cload(A.coefs + k);
   if (k >= 1) {
@@ -370,8 +377,48 @@ __device__ __forceinline__ uint32_t uni(uint32_t v) {
 
 // What the blocks of a team share about the job in hand.
 struct TeamShared {
-  uint32_t idx, n, bar, slot, ok, job, seg;
+  uint32_t idx, n, bar, slot, ok, job, seg, pad[9];
+  double red[2 * kTeamWaves];  // the waves' dots of a step
 };
+
+// KPM dots of one step.  FP64: <T_{j-1}, T_{j-1}> and <T_j, T_{j-1}>, from which
+// mu_{2j-2} and mu_{2j-1} follow (2 T_m T_n = T_{m+n} + T_{m-n}): half the steps of
+// the direct form.  FP32: <x, x> and <x, T_j>, because there the identity's
+// rounding can exceed the direct form's.
+struct TeamDots {
+  double a = 0.0, b = 0.0;
+  template <typename T>
+  __device__ __forceinline__ void add(pair_t<T> x, pair_t<T> own, pair_t<T> o, bool ok, bool two) {
+    if constexpr (sizeof(T) == 8) x = own;
+    const double a0 = (double)x[0] * (double)x[0], b0 = (double)x[0] * (double)o[0];
+    const double a1 = (double)x[1] * (double)x[1], b1 = (double)x[1] * (double)o[1];
+    a += ok ? a0 : 0.0;
+    b += ok ? b0 : 0.0;
+    a += two ? a1 : 0.0;
+    b += two ? b1 : 0.0;
+  }
+  // the wave's sums to LDS
+  __device__ __forceinline__ void park(TeamShared& sh) {
+    for (int o = 32; o > 0; o >>= 1) {
+      a += __shfl_down(a, o, 64);
+      b += __shfl_down(b, o, 64);
+    }
+    if ((threadIdx.x & 63u) == 0) {
+      sh.red[2 * (threadIdx.x >> 6)] = a;
+      sh.red[2 * (threadIdx.x >> 6) + 1] = b;
+    }
+  }
+};
+// The block's sums of step j (all waves parked): written by two threads of wave 1.
+__device__ __forceinline__ void team_dots_out(const TeamArgs& A, const TeamShared& sh, int j,
+                                              int col, uint32_t idx) {
+  if (threadIdx.x >= 64u && threadIdx.x < 66u) {
+    const uint32_t w = threadIdx.x - 64u;
+    double t = 0.0;
+    for (int i = 0; i < kTeamWaves; ++i) t += sh.red[2 * i + w];
+    A.dots[((int64_t)(2 * (j - 1) + (int)w) * A.ncols + col) * kTeamUnits + idx] = t;
+  }
+}
 
 // Both halves of the barrier around `between` (this block's own LDS update).
 template <class F>
@@ -404,7 +451,7 @@ __device__ __forceinline__ bool team_next(const TeamArgs& A, TeamShared& sh, Tea
 }
 
 // The streaming form of one column (any team size, any D).
-template <typename T, int NQ, int NC, bool UNI>
+template <typename T, int NQ, int NC, bool UNI, bool KPM>
 __device__ bool stream_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me, int col,
                               char* slot) {
   constexpr uint32_t sz = sizeof(T);
@@ -419,14 +466,17 @@ __device__ bool stream_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me, 
   double* Y = A.Y + (int64_t)col * A.ldy;
   const __amdgpu_buffer_rsrc_t x32 = rsrc_of(slot + 2 * (int64_t)bytes, bytes);
   lwrite<T>(rows - sz, (T)0);
-  int k = A.order;
-  // b2 = c_K X (and X in the arithmetic's type), then the steps K-1 .. 0
-  for (bool first = true; k >= 0; --k, first = false) {
-    const TeamCoef<T> f = team_coef<T>(A, k);
-    const int par = (A.order - k) & 1;
+  const int steps = A.order;
+  const double fx = KPM ? A.colscale[col] : 1.0;
+  TeamDots dots;
+  // the first vector (c_K X, or T_0 = x), then the steps 1 .. order
+  for (int j = 0; j <= steps; ++j) {
+    const bool first = j == 0;
+    const TeamCoef<T> f = first && KPM ? TeamCoef<T>{(T)1, (T)0, (T)0} : team_coef<T, KPM>(A, j);
+    const int par = j & 1;
     const __amdgpu_buffer_rsrc_t out = rsrc_of(slot + par * (int64_t)bytes, bytes);  // b3, then b1
     const __amdgpu_buffer_rsrc_t b2 = rsrc_of(slot + (1 - par) * (int64_t)bytes, bytes);
-    const bool hasB3 = k <= A.order - 2;
+    const bool hasB3 = j >= 2;
     for (int u = (int)me.idx; u < kTeamUnits; u += (int)me.n) {
       const int s1 = cload(A.uofs + u + 1);
       int at = cload(A.uofs + u);
@@ -452,7 +502,7 @@ __device__ bool stream_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me, 
           const uint32_t i = g.i0 + 2u * ln, vo = i * sz;
           const int64_t row = (int64_t)g.seg0 + i;
           pt x;
-          if (first || !A.has_x) x = x_pair<T>(A, X, row, two);
+          if (first || !A.has_x) x = x_pair<T>(A, X, row, two, fx);
           else x = bload<pt>(x32, vo, g.pos * sz);
           pt o = f.cx * x;
           if (first) {
@@ -465,12 +515,14 @@ __device__ bool stream_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me, 
             low_sum<T, NQ, NC, UNI>(bs, tab, rows - sz);
             outer_sum<T, NQ, NC, UNI>(bs, A, g, vo, tab, bytes, b2);
             const pt hs = bs.value();
-            o += f.ch * (d * lread<pt>(rows + vo) + hs);
+            const pt own = lread<pt>(rows + vo);
+            o += f.ch * (d * own + hs);
             o += f.cb * b3;
+            if constexpr (KPM) dots.add<T>(x, own, o, ok, ok && two);
           }
-          if (k > 0) {
+          if (j < steps) {
             bstore<pt>(o, out, ok ? vo : bytes, g.pos * sz);
-          } else if (ok) {
+          } else if (!KPM && ok) {
             y_pair<T>(A, Y, row, two, o);
           }
         }
@@ -482,7 +534,18 @@ __device__ bool stream_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me, 
         __syncthreads();
       }
     }
-    if (k > 0 && !team_step_end(A, sh, me, false, [] {})) return false;
+    if (KPM && !first) {
+      dots.park(sh);
+      dots = TeamDots{};
+    }
+    if (j < steps && !team_step_end(A, sh, me, false, [&] {
+          if (KPM && !first) team_dots_out(A, sh, j, col, me.idx);
+        }))
+      return false;
+  }
+  if constexpr (KPM) {
+    __syncthreads();
+    team_dots_out(A, sh, steps, col, me.idx);
   }
   return true;
 }
@@ -533,7 +596,7 @@ __device__ __forceinline__ uint32_t lrec_word(const uint32_t* rec, int k, uint32
 // before each segment.  Segments of the same block are read from LDS, the others
 // from memory, all of a group's loads before its first sum.  LDS: class tables,
 // records, rows, spare elements.
-template <typename T, int NQ, int NC, bool UNI, int R>
+template <typename T, int NQ, int NC, bool UNI, bool KPM, int R>
 __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me,
                                                 int col, char* slot) {
   constexpr uint32_t sz = sizeof(T);
@@ -559,7 +622,8 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
   auto last_of = [&](const LRec& c) { return ((c[kRecCnt] & 0xFFu) - 1u) >> 1; };
   const uint32_t spare = A.rows_lds - 4u * sz;  // takes the writes of lanes without a row
   pt x[R], p[R], d[kDiagReg ? R : 1];
-  const TeamCoef<T> fk = team_coef<T>(A, A.order);
+  const T fk = KPM ? (T)1 : (T)cload(A.coefs + A.order);
+  const double fx = KPM ? A.colscale[col] : 1.0;
   __amdgpu_buffer_rsrc_t out = rsrc_of(slot, bytes);
   __amdgpu_buffer_rsrc_t in = rsrc_of(slot + bytes, bytes);
 #pragma unroll
@@ -571,15 +635,17 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
       const uint32_t last = last_of(c), ln = lane < last ? lane : last;
       const int64_t row = (int64_t)c[kRecRow] + 2u * ln;
       const bool two = 2u * ln + 1u < (c[kRecCnt] & 0xFFu);
-      x[r] = x_pair<T>(A, X, row, two);
+      x[r] = x_pair<T>(A, X, row, two, fx);
       if constexpr (kDiagReg) d[r] = d_pair<T>(A, row, two);
-      p[r] = fk.cx * x[r];  // (the new vector; it moves to LDS behind the barrier)
+      p[r] = fk * x[r];  // (the new vector; it moves to LDS behind the barrier)
       if constexpr (NC > 0)
         bstore<pt>(p[r], out, lane <= last ? c[kRecI0] + 2u * ln * sz : bytes, c[kRecPos]);
     }
   }
-  for (int k = A.order - 1; k >= 0; --k) {
-    const TeamCoef<T> f = team_coef<T>(A, k);
+  TeamDots dots;
+  for (int j = 1; j <= A.order; ++j) {
+    const bool last_step = j == A.order;
+    const TeamCoef<T> f = team_coef<T, KPM>(A, j);
     int zero;  // (opaque: the R conditions are not hoisted into saved masks)
     asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
     left = mine + zero;
@@ -593,8 +659,9 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
                                       ? c[kRecZero] + sz + c[kRecI0] + 2u * lane * sz : spare;
               const pt t = lread<pt>(at);
               lwrite<pt>(at, p[r]);
-              p[r] = k == A.order - 1 ? (pt)(T)0 : t;  // (LDS is another column's then)
+              p[r] = j == 1 ? (pt)(T)0 : t;  // (LDS is another column's then)
             }
+          if (KPM && j > 1) team_dots_out(A, sh, j - 1, col, me.idx);
         }))
       return false;
     const __amdgpu_buffer_rsrc_t t = in;
@@ -688,23 +755,33 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
         }
       }
       const pt hs = bs.value();
-      pt o = f.cx * x[r];
-      o += f.ch * (dg * own + hs);
+      pt o = f.ch * (dg * own + hs);
+      if constexpr (!KPM) o += f.cx * x[r];
       o += f.cb * p[r];
       p[r] = o;
-      if (k > 0) {
+      if constexpr (KPM)
+        dots.add<T>(x[r], own, o, lane <= last, lane <= last && 2u * ln + 1u < (cnt & 0xFFu));
+      if (!last_step) {
         if constexpr (NC > 0) bstore<pt>(o, out, lane <= last ? vo : bytes, c[kRecPos]);
-      } else if (lane <= last) {
+      } else if (!KPM && lane <= last) {
         y_pair<T>(A, Y, (int64_t)c[kRecRow] + 2u * ln, 2u * ln + 1u < (cnt & 0xFFu), o);
       }
     }
+    if constexpr (KPM) {
+      dots.park(sh);
+      dots = TeamDots{};
+    }
+  }
+  if constexpr (KPM) {
+    __syncthreads();
+    team_dots_out(A, sh, A.order, col, me.idx);
   }
   return true;
 }
 
 // R = 0: the streaming form only.  Dynamic LDS: class tables (at offset 0, so
 // that offsets need no base), then the form's own area, then TeamShared.
-template <typename T, int NQ, int NC, bool UNI, int R>
+template <typename T, int NQ, int NC, bool UNI, bool KPM, int R>
 __global__ __launch_bounds__(kTeamThreads) void chain_team_kernel(const TeamArgs A) {
   TeamShared& sh = *reinterpret_cast<TeamShared*>(team_lds + A.rows_lds);
   TeamPlace me{};
@@ -756,12 +833,12 @@ __global__ __launch_bounds__(kTeamThreads) void chain_team_kernel(const TeamArgs
     if (col >= (uint32_t)A.ncols) return;
     bool ok;
     if constexpr (R > 0 && NC == 0) {
-      ok = resident_column<T, NQ, NC, UNI, R>(A, sh, me, (int)col, work);
+      ok = resident_column<T, NQ, NC, UNI, KPM, R>(A, sh, me, (int)col, work);
     } else if constexpr (R > 0) {
-      ok = me.n == (uint32_t)A.T ? resident_column<T, NQ, NC, UNI, R>(A, sh, me, (int)col, work)
-                                 : stream_column<T, NQ, NC, UNI>(A, sh, me, (int)col, work);
+      ok = me.n == (uint32_t)A.T ? resident_column<T, NQ, NC, UNI, KPM, R>(A, sh, me, (int)col, work)
+                                 : stream_column<T, NQ, NC, UNI, KPM>(A, sh, me, (int)col, work);
     } else {
-      ok = stream_column<T, NQ, NC, UNI>(A, sh, me, (int)col, work);
+      ok = stream_column<T, NQ, NC, UNI, KPM>(A, sh, me, (int)col, work);
     }
     if (!ok) return;
     if (threadIdx.x == 0 && me.idx == 0) (void)team_add(&A.ctl->done, 1u);
@@ -1194,7 +1271,7 @@ TeamTables* team_build(const ChainParams& ref, const uint32_t* C, const uint32_t
 }
 
 // --------------------------------------------------------------- the plan
-constexpr size_t kTeamLds = 160 * 1024 - 64;  // the rest: TeamShared
+constexpr size_t kTeamLds = 160 * 1024 - sizeof(TeamShared);
 
 static size_t team_table_bytes(const TeamTables* t) { return (size_t)8 * t->NQ * tab_rows(t->NC); }
 // Dynamic LDS of the resident form: tables, records, rows with zero slots, and
@@ -1242,6 +1319,8 @@ static double per_step_us(int64_t D, int dtype, int ncols) {
   return std::max(5.0, mb / (mb > 512 ? 1.4 : 2.6));
 }
 
+int team_kpm_steps(int dtype, int N);
+
 // Blocks per column of the fastest team form, and its time.
 int team_best(const pf_op* op, int dtype, int ncols, double* us) {
   const TeamTables* t = op->team;
@@ -1262,15 +1341,12 @@ int team_best(const pf_op* op, int dtype, int ncols, double* us) {
 // Below this order the begin and end launches cost what the steps save.
 constexpr int kTeamMinOrder = 8;
 
-int team_plan(const pf_op* op, int dtype, int polytype, int order, const double* X, int64_t ldx,
-              const double* Y, int64_t ldy, int ncols) {
+// Blocks per column for `order` steps on ncols columns, or 0.  `gain`: the steps
+// that the per-step launches take for one of these.
+static int team_choose(const pf_op* op, int dtype, int order, int ncols, int gain) {
   const TeamTables* t = op->team;
   const TuneCfg& f = op->force;
-  if (!t || order < 1 || polytype == PF_TAYLOR || f.team == 0) return 0;
-  // a column's result may replace that column of X, but no other
-  const double* xe = X + (ncols - 1) * ldx + op->D;
-  const double* ye = Y + (ncols - 1) * ldy + op->D;
-  if (X < ye && Y < xe && !(X == Y && ldx == ldy)) return 0;
+  if (!t || order < 1 || f.team == 0) return 0;
   if (f.team > 0) return t->NC == 0 ? 1 : f.team;
   // forced launch knobs are those of the per-step kernels
   if (f.V || f.xcd >= 0 || f.nt >= 0 || f.pb >= 0 || f.wide >= 0 || f.occ >= 0 || f.part >= 0)
@@ -1278,84 +1354,91 @@ int team_plan(const pf_op* op, int dtype, int polytype, int order, const double*
   if (order < kTeamMinOrder) return 0;
   // measured by the autotuner, else by the rule (by chunks of columns there)
   const auto it = op->tuned.find({dtype, ncols});
-  if (it != op->tuned.end() && it->second.team >= 0) return it->second.team;
+  if (it != op->tuned.end() && (it->second.team > 0 || (it->second.team == 0 && gain == 1)))
+    return it->second.team;
   double us;
   const int T = team_best(op, dtype, ncols, &us);
-  return us < 0.95 * per_step_us(op->D, dtype, ncols) ? T : 0;
+  return us < 0.95 * gain * per_step_us(op->D, dtype, ncols) ? T : 0;
 }
 
-size_t team_work_bytes(const pf_op* op, int dtype, int order, int ncols, int T, int* nslots,
-                       size_t* slot) {
-  const size_t sz = dtype == PF_F64 ? 8 : 4;
-  const size_t vec = (size_t)op->team->elems * sz;
-  *nslots = std::min(ncols, 8 * (32 / T));
-  *slot = (dtype == PF_F64 && !op->team->perm ? 2 : 3) * vec;
-  return ((sizeof(TeamCtl) + 255) & ~(size_t)255) + (((size_t)(order + 1) * 8 + 255) & ~(size_t)255) +
-         *nslots * *slot;
+int team_plan(const pf_op* op, int dtype, int polytype, int order, const double* X, int64_t ldx,
+              const double* Y, int64_t ldy, int ncols) {
+  if (polytype == PF_TAYLOR) return 0;
+  // a column's result may replace that column of X, but no other
+  const double* xe = X + (ncols - 1) * ldx + op->D;
+  const double* ye = Y + (ncols - 1) * ldy + op->D;
+  if (X < ye && Y < xe && !(X == Y && ldx == ldy)) return 0;
+  return team_choose(op, dtype, order, ncols, 1);
 }
 
-template <typename T, int NQ, int NC, bool UNI, int R>
+// FP64 moments take half the steps here (TeamDots), so the team wins far above the
+// sizes where the filter's does: 32 probes, N = 250, L = 20: 18.0 -> 3.6 ms (team of
+// 16); 16 probes, L = 22: 9.1 -> 2.9 ms at N = 60 (streamed); FP32, the same steps:
+// L = 20 8.0 -> 5.3 ms, L = 18 2.9 -> 1.5 ms (team of 8).
+int team_kpm_plan(const pf_op* op, int dtype, int N, int ncols) {
+  return team_choose(op, dtype, team_kpm_steps(dtype, N), ncols, dtype == PF_F64 ? 2 : 1);
+}
+
+static size_t team_align(size_t n) { return (n + 255) & ~(size_t)255; }
+
+size_t team_work_bytes(const pf_op* op, int dtype, int order, int ncols, int T) {
+  const size_t vec = (size_t)op->team->elems * (dtype == PF_F64 ? 8 : 4);
+  return team_align(sizeof(TeamCtl)) + team_align((size_t)(order + 1) * 8) +
+         std::min(ncols, 8 * (32 / T)) * 3 * vec;
+}
+
+template <typename T, int NQ, int NC, bool UNI, bool KPM, int R>
 static void team_launch(const TeamArgs& A, int grid, size_t lds, hipStream_t st) {
-  auto* k = chain_team_kernel<T, NQ, NC, UNI, R>;
+  auto* k = chain_team_kernel<T, NQ, NC, UNI, KPM, R>;
   PF_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kTeamThreads), lds, st, A);
   PF_HIP(hipGetLastError());
 }
 
-template <typename T, int NQ, int NC, bool UNI>
+template <typename T, int NQ, int NC, bool UNI, bool KPM>
 static void team_launch_r(const TeamArgs& A, int R, int grid, size_t lds, hipStream_t st) {
-  if (R == 1) return team_launch<T, NQ, NC, UNI, 1>(A, grid, lds, st);
-  if (R == 2) return team_launch<T, NQ, NC, UNI, 2>(A, grid, lds, st);
+  if (R == 1) return team_launch<T, NQ, NC, UNI, KPM, 1>(A, grid, lds, st);
+  if (R == 2) return team_launch<T, NQ, NC, UNI, KPM, 2>(A, grid, lds, st);
   if constexpr (NC > 0) {
-    if (R == 4) return team_launch<T, NQ, NC, UNI, 4>(A, grid, lds, st);
+    if (R == 4) return team_launch<T, NQ, NC, UNI, KPM, 4>(A, grid, lds, st);
     if constexpr (NQ == 3 || sizeof(T) == 4)
-      if (R == 7) return team_launch<T, NQ, NC, UNI, 7>(A, grid, lds, st);
+      if (R == 7) return team_launch<T, NQ, NC, UNI, KPM, 7>(A, grid, lds, st);
     if constexpr (NQ == 3 && sizeof(T) == 4)
-      if (R == 13) return team_launch<T, NQ, NC, UNI, 13>(A, grid, lds, st);
-    if (R == 0) return team_launch<T, NQ, NC, UNI, 0>(A, grid, lds, st);
+      if (R == 13) return team_launch<T, NQ, NC, UNI, KPM, 13>(A, grid, lds, st);
+    if (R == 0) return team_launch<T, NQ, NC, UNI, KPM, 0>(A, grid, lds, st);
   }
   throw Error{PF_ERR_UNSUPPORTED, "team filter: no kernel for this plan"};
 }
 
-template <typename T>
+template <typename T, bool KPM>
 static void team_launch_t(const TeamTables* t, const TeamArgs& A, int R, int grid, size_t lds,
                           hipStream_t st) {
   if (t->NC == 0) {
-    if (t->NQ == 3) team_launch_r<T, 3, 0, true>(A, R, grid, lds, st);
-    else team_launch_r<T, 6, 0, false>(A, R, grid, lds, st);
+    if (t->NQ == 3) team_launch_r<T, 3, 0, true, KPM>(A, R, grid, lds, st);
+    else team_launch_r<T, 6, 0, false, KPM>(A, R, grid, lds, st);
   } else {
-    if (t->NQ == 3) team_launch_r<T, 3, 2, true>(A, R, grid, lds, st);
-    else team_launch_r<T, 6, 6, false>(A, R, grid, lds, st);
+    if (t->NQ == 3) team_launch_r<T, 3, 2, true, KPM>(A, R, grid, lds, st);
+    else team_launch_r<T, 6, 6, false, KPM>(A, R, grid, lds, st);
   }
 }
 
-void team_filter(pf_op* op, int dtype, int polytype, const double* coeffs, int order,
-                 const double* X, int64_t ldx, double* Y, int64_t ldy, int ncols, int T,
-                 void* work, hipStream_t st) {
+// One launch over all columns: the filter (dots null) or the KPM recurrence of
+// `order` steps.  work: control words, coefficients, the teams' vectors.
+static void team_run(pf_op* op, int dtype, TeamArgs A, int T, void* work, size_t coef_bytes,
+                     hipStream_t st) {
   const TeamTables* t = op->team;
   const int w = dtype == PF_F64 ? 0 : 1;
   const size_t sz = dtype == PF_F64 ? 8 : 4;
-  int nslots;
-  size_t slot;
-  team_work_bytes(op, dtype, order, ncols, T, &nslots, &slot);
+  const bool kpm = A.dots != nullptr;
   char* p = (char*)work;
-  TeamCtl* ctl = (TeamCtl*)p;
-  p += (sizeof(TeamCtl) + 255) & ~(size_t)255;
-  double* cdev = (double*)p;
-  p += ((size_t)(order + 1) * 8 + 255) & ~(size_t)255;
-  for (int at = 0; at <= order; at += kCoefChunk) {
-    TeamCoefs c;
-    const int n = std::min(kCoefChunk, order + 1 - at);
-    std::memcpy(c.c, coeffs + at, n * sizeof(double));
-    hipLaunchKernelGGL(team_begin_kernel, dim3(1), dim3(1024), 0, st, at ? nullptr : ctl, cdev, at,
-                       n, c);
-    PF_HIP(hipGetLastError());
-  }
+  A.ctl = (TeamCtl*)p;
+  p += team_align(sizeof(TeamCtl));
+  A.coefs = (const double*)p;
+  p += team_align(coef_bytes);
   int lt = 0;
   while ((1 << lt) < T) ++lt;
   const int R = team_resident(t, dtype, lt);
   const Affine af = op->affine(true);
-  TeamArgs A{};
   A.tab = t->tab[w];
   A.grp = t->grp;
   A.rec = t->rec[lt];
@@ -1370,40 +1453,128 @@ void team_filter(pf_op* op, int dtype, int polytype, const double* coeffs, int o
   A.sgrp = t->sgrp;
   A.ntab = t->ntab;
   A.T = T;
-  A.order = order;
-  A.polytype = polytype;
-  A.ncols = ncols;
   A.maxseg = t->maxseg;
   A.elems = (uint32_t)t->elems;
   A.tab_lds = (uint32_t)team_table_bytes(t);
   A.diag = t->diag ? t->diag : op->diag;
+  A.perm = t->perm;
   A.scale = af.scale;
   A.shift = af.shift;
-  A.X = X;
-  A.ldx = ldx;
-  A.Y = Y;
-  A.ldy = ldy;
   A.work = p;
-  A.slot_bytes = (int64_t)slot;
-  A.nslots = nslots;
-  A.has_x = slot > 2 * (size_t)t->elems * sz;
-  A.perm = t->perm;
-  A.ctl = ctl;
-  A.coefs = cdev;
+  // the streaming form keeps its own copy of X where the caller's is not FP64 in
+  // the team's row order
+  A.has_x = dtype != PF_F64 || t->perm || kpm;
+  A.slot_bytes = (int64_t)(3 * (size_t)t->elems * sz);
+  A.nslots = std::min(A.ncols, 8 * (32 / T));
   const int cus = std::max(1, op->h->prop.multiProcessorCount);
   const int nxcd = std::max(1, cus / 32);
   const int grid = std::max(T, cus / nxcd * nxcd);
   A.expect = grid / nxcd;
   size_t lds = R ? team_resident_lds(t, lt, sz) : team_table_bytes(t);
   if (t->NC > 0) lds = std::max(lds, team_stream_lds(t, sz));
-
   lds = (lds + 31) & ~(size_t)31;
   A.rows_lds = (uint32_t)lds;
-  lds += 64;  // TeamShared
-  if (dtype == PF_F64) team_launch_t<double>(t, A, R, grid, lds, st);
-  else team_launch_t<float>(t, A, R, grid, lds, st);
+  lds += sizeof(TeamShared);
+  if (kpm) {
+    if (dtype == PF_F64) team_launch_t<double, true>(t, A, R, grid, lds, st);
+    else team_launch_t<float, true>(t, A, R, grid, lds, st);
+  } else {
+    if (dtype == PF_F64) team_launch_t<double, false>(t, A, R, grid, lds, st);
+    else team_launch_t<float, false>(t, A, R, grid, lds, st);
+  }
+}
+
+void team_filter(pf_op* op, int dtype, int polytype, const double* coeffs, int order,
+                 const double* X, int64_t ldx, double* Y, int64_t ldy, int ncols, int T,
+                 void* work, hipStream_t st) {
+  TeamCtl* ctl = (TeamCtl*)work;
+  double* cdev = (double*)((char*)work + team_align(sizeof(TeamCtl)));
+  for (int at = 0; at <= order; at += kCoefChunk) {
+    TeamCoefs c;
+    const int n = std::min(kCoefChunk, order + 1 - at);
+    std::memcpy(c.c, coeffs + at, n * sizeof(double));
+    hipLaunchKernelGGL(team_begin_kernel, dim3(1), dim3(1024), 0, st, at ? nullptr : ctl, cdev, at,
+                       n, c);
+    PF_HIP(hipGetLastError());
+  }
+  TeamArgs A{};
+  A.order = order;
+  A.polytype = polytype;
+  A.ncols = ncols;
+  A.X = X;
+  A.ldx = ldx;
+  A.Y = Y;
+  A.ldy = ldy;
+  team_run(op, dtype, A, T, work, (size_t)(order + 1) * 8, st);
   hipLaunchKernelGGL(team_end_kernel, dim3(256), dim3(256), 0, st, ctl, (uint32_t)ncols, Y, ldy,
                      op->D);
+  PF_HIP(hipGetLastError());
+}
+
+// ------------------------------------------------------------------ KPM
+__global__ void team_zero_kernel(double* p, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    p[i] = 0.0;
+}
+// dots[step][which] summed over columns and blocks in a fixed order; NaN when a
+// column was not finished
+__global__ __launch_bounds__(256) void team_dots_kernel(const double* __restrict__ dots, int ncols,
+                                                        const TeamCtl* ctl,
+                                                        double* __restrict__ sums) {
+  __shared__ double red[4];
+  const double* p = dots + (int64_t)blockIdx.x * ncols * kTeamUnits;
+  double t = 0.0;
+  for (int i = threadIdx.x; i < ncols * kTeamUnits; i += 256) t += p[i];
+  t = block_sum_256(t, red);
+  if (threadIdx.x == 0)
+    sums[blockIdx.x] = ctl->done == (uint32_t)ncols && ctl->abort == 0 ? t : __builtin_nan("");
+}
+// mu[n] += the moments of one chunk of columns from its dots
+__global__ void team_moments_kernel(const double* __restrict__ sums, int f64, int N,
+                                    double* __restrict__ mu) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= N) return;
+  double v;
+  if (f64) {  // sums[2j] = <T_j, T_j>, sums[2j+1] = <T_{j+1}, T_j>
+    v = sums[n];
+    if (n >= 2) v = 2.0 * v - sums[n & 1];
+  } else {    // sums[2j+1] = <x, T_{j+1}>
+    v = n == 0 ? sums[0] : sums[2 * n - 1];
+  }
+  mu[n] += v;
+}
+
+int team_kpm_steps(int dtype, int N) { return dtype == PF_F64 ? (N + 1) / 2 : N - 1; }
+
+size_t team_kpm_bytes(const pf_op* op, int dtype, int N, int ncols, int T) {
+  const size_t steps = team_kpm_steps(dtype, N);
+  return team_work_bytes(op, dtype, 0, ncols, T) + team_align(2 * steps * ncols * kTeamUnits * 8) +
+         team_align(2 * steps * 8);
+}
+
+void team_kpm(pf_op* op, int dtype, int N, const double* X, int64_t ldx, int ncols,
+              const double* colscale, double* mu, int T, void* work, hipStream_t st) {
+  const int steps = team_kpm_steps(dtype, N);
+  TeamCtl* ctl = (TeamCtl*)work;
+  double* dots = (double*)((char*)work + team_work_bytes(op, dtype, 0, ncols, T));
+  const int64_t n = (int64_t)2 * steps * ncols * kTeamUnits;
+  double* sums = (double*)((char*)dots + team_align(n * 8));
+  TeamCoefs none{};
+  hipLaunchKernelGGL(team_begin_kernel, dim3(1), dim3(1024), 0, st, ctl, nullptr, 0, 0, none);
+  hipLaunchKernelGGL(team_zero_kernel, dim3(512), dim3(256), 0, st, dots, n);
+  PF_HIP(hipGetLastError());
+  TeamArgs A{};
+  A.order = steps;
+  A.ncols = ncols;
+  A.X = X;
+  A.ldx = ldx;
+  A.colscale = colscale;
+  A.dots = dots;
+  team_run(op, dtype, A, T, work, 8, st);
+  hipLaunchKernelGGL(team_dots_kernel, dim3(2 * steps), dim3(256), 0, st, dots, ncols, ctl, sums);
+  hipLaunchKernelGGL(team_moments_kernel, dim3((N + 255) / 256), dim3(256), 0, st, sums,
+                     dtype == PF_F64, N, mu);
   PF_HIP(hipGetLastError());
 }
 

@@ -10,6 +10,7 @@ import scipy.sparse as sp
 import torch
 
 from oracle import clenshaw as oc
+from oracle import dos as odos
 from oracle import models as om
 
 pytestmark = pytest.mark.gpu
@@ -106,3 +107,20 @@ def test_team_filter_more_couplings_than_classes(dev):
     c = oc.filter_coefficients(0.3, 25)
     Y = dev.to_host(op.filter(c, dev.to_device(X)))
     assert _rel(Y, oc.clenshaw_apply(lambda Z: (H / g) @ Z, c, X)) < 1e-12
+
+
+# moments are averages of products of such vectors: the per-step moments' bounds
+@pytest.mark.parametrize("dtype,tol", [("f64", 1e-12), ("f32", 2e-4)])
+@pytest.mark.parametrize("case", CASES[1:], ids=[c[0] for c in CASES[1:]])
+def test_team_moments_match_oracle(dev, case, dtype, tol):
+    """Every moment, odd and even counts of them: FP64 takes two per step."""
+    name, L, Lup, J2, boundary, s, teams = case
+    op, Ht = _chain(dev, L, Lup, J2, boundary, len(name))
+    P = np.random.default_rng(L).standard_normal((op.D, s))
+    Pd = dev.to_device(P)
+    for N in (2, 3, 40):
+        ref = odos.dos_moments(lambda v: Ht @ v, N, P)
+        for T in teams:
+            op.set_tuning(team=T)
+            mu = op.kpm_moments(N, Pd, dtype=dtype)
+            assert np.max(np.abs(mu - ref)) / op.D < tol, (N, T)
