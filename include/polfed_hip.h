@@ -357,13 +357,18 @@ enum {
                                   block's rows (256 / (ncols / vec) x rows per
                                   lane) hold <= 32 KiB in FP64; ignored otherwise
                                   (default 0)                                     */
-  PF_BATCH_ROW_VECTORS = 8     /* 1 or 2: with ncols = 1, a lane takes 16 bytes
+  PF_BATCH_ROW_VECTORS = 8,    /* 1 or 2: with ncols = 1, a lane takes 16 bytes
                                   of consecutive rows (4 FP32 or 2 FP64) per load,
                                   1 or 2 such vectors at a time, and a block
                                   1024 x rows per lane rows, staged in LDS; used
                                   when vec = 1 and rows per lane is 1, 2 or 4 (2
                                   or 4 for the value 2), ignored otherwise
                                   (default 0)                                     */
+  PF_BATCH_TEAM = 9            /* one launch for the whole application, this many
+                                  blocks (1, 2, 4, .. 32) per column; 0: the
+                                  per-step forms; -1: by a rule (default).  The
+                                  autotuner sets it; setting a key 3 .. 8 sets it
+                                  to 0                                            */
 };
 /* Launch settings of the batch.  No reference counterpart. */
 int pf_batch_set_tuning(pf_batch* b, int32_t key, int32_t value);

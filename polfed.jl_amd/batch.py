@@ -5,8 +5,9 @@ once per Lanczos iteration (``clenshaw(transform, W, V, b, ::GPU,
 ::NoParallel)``, src/Polfed/Algorithm/SpectralTransformation/ParallelizationClenshaw.jl:41-51).
 A ``QSunBatch`` applies the filters of many instances -- disorder
 realizations of possibly different sizes, each with its own polynomial and
-rescaling -- as one multi-instance kernel launch per Clenshaw step, replayed
-from a captured HIP graph.
+rescaling -- in one launch, each column on a team of blocks for all its steps, or
+where that does not fit as one multi-instance kernel launch per Clenshaw step,
+replayed from a captured HIP graph.
 """
 from __future__ import annotations
 
@@ -24,7 +25,8 @@ from .operators import QSunOperator, _dtype
 _TUNE = {"graph": _lib.PF_BATCH_GRAPH, "graph_steps": _lib.PF_BATCH_GRAPH_STEPS,
          "vec": _lib.PF_BATCH_VEC, "rows_per_lane": _lib.PF_BATCH_ROWS_PER_LANE,
          "xcd": _lib.PF_BATCH_XCD, "grain_shuffle": _lib.PF_BATCH_GRAIN_SHUFFLE,
-         "lds_rows": _lib.PF_BATCH_LDS_ROWS, "row_vectors": _lib.PF_BATCH_ROW_VECTORS}
+         "lds_rows": _lib.PF_BATCH_LDS_ROWS, "row_vectors": _lib.PF_BATCH_ROW_VECTORS,
+         "team": _lib.PF_BATCH_TEAM}
 
 
 class QSunBatch:
@@ -110,7 +112,8 @@ class QSunBatch:
 
     def set_tuning(self, **kw) -> None:
         """graph (0/1), graph_steps, vec, rows_per_lane, xcd, grain_shuffle (0/1),
-        lds_rows (0/1), row_vectors (0/1/2)."""
+        lds_rows (0/1), row_vectors (0/1/2); team (-1/0/1/2/4/.../32): blocks per
+        column of the one-launch form, 0 for the per-step forms, -1 for a rule."""
         for k, v in kw.items():
             if k not in _TUNE:
                 raise ValueError(f"unknown batch tuning key {k!r}")

@@ -14,7 +14,7 @@ import tempfile
 PKG = pathlib.Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OUT = PKG / "lib" / "libpolfed_hip.so"
-SOURCES = ["ops.hip", "team.hip", "batch.hip", "packed.hip", "dense.hip", "capi.cpp"]
+SOURCES = ["ops.hip", "team.hip", "qteam.hip", "batch.hip", "packed.hip", "dense.hip", "capi.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 FLAGS = [

@@ -24,6 +24,9 @@
 // (the grain block and the flips that stay inside the block's aligned row
 // range read from LDS), and row vectors for one column (a lane takes 16
 // bytes of consecutive rows per load; blocks staged in LDS as well).
+//
+// Where every instance fits, the whole application runs as one launch instead,
+// each instance's column on a team of blocks for all its steps (qteam.hip).
 
 #include <algorithm>
 #include <cmath>
@@ -82,15 +85,6 @@ struct BatchArgs {
 
 // LDS form: the block's rows of b2 (dynamic shared memory, rows x row stride)
 extern __shared__ __align__(16) char batch_rows[];
-
-__device__ __forceinline__ void poly_ab_dev(int type, int k, double& alpha, double& beta_k) {
-  switch (type) {
-    case PF_LEGENDRE: alpha = (2.0 * k + 1) / (k + 1); beta_k = -(double)k / (k + 1); break;
-    case PF_HERMITE: alpha = 2.0; beta_k = -2.0 * k; break;
-    case PF_TAYLOR: alpha = 1.0; beta_k = 0.0; break;
-    default: alpha = 2.0; beta_k = -1.0; break;  // Chebyshev
-  }
-}
 
 // Buffer slot written at local step g (rotation (3,1,2) of the recurrence).
 __device__ __forceinline__ int rot_slot(int g) { return (3 - g % 3) % 3; }
@@ -624,9 +618,16 @@ struct pf_batch {
   DevBuf insts, dyn, blk0d, coefs, kstate, bufs;
   // tuning
   int V = 1, rpt = 1, xcd = 1, use_graph = 1, gsteps = 96, shfl = 1, lds = 0, rv = 0;
+  // one-launch form: blocks per column, 0 the per-step forms, -1 by the rule;
+  // the operators' records and the control words
+  int team = -1;
+  bool team_forced = false;
+  DevBuf trecs, tctl;
   // pinned staging of the per-application records; the event marks the end
   // of the last copy out of it
   BatchDyn* hdyn = nullptr;
+  QsunJob* hjobs = nullptr;
+  DevBuf jobs;
   hipEvent_t dyn_done = nullptr;
   bool dyn_pending = false;
   // graph state
@@ -677,13 +678,15 @@ struct pf_batch {
       graph[m] = nullptr;
     }
   }
+  void stage_ready() {
+    if (!dyn_done) PF_HIP(hipEventCreateWithFlags(&dyn_done, hipEventDisableTiming));
+    if (dyn_pending) PF_HIP(hipEventSynchronize(dyn_done));
+    dyn_pending = false;
+  }
   // Stage per-application records and copy them to the device on st.
   void upload_dyn(const std::vector<BatchDyn>& dy, hipStream_t st) {
-    if (!hdyn) {
-      PF_HIP(hipHostMalloc(reinterpret_cast<void**>(&hdyn), n * sizeof(BatchDyn)));
-      PF_HIP(hipEventCreateWithFlags(&dyn_done, hipEventDisableTiming));
-    }
-    if (dyn_pending) PF_HIP(hipEventSynchronize(dyn_done));
+    if (!hdyn) PF_HIP(hipHostMalloc(reinterpret_cast<void**>(&hdyn), n * sizeof(BatchDyn)));
+    stage_ready();
     std::memcpy(hdyn, dy.data(), n * sizeof(BatchDyn));
     PF_HIP(hipMemcpyAsync(dyn.p, hdyn, n * sizeof(BatchDyn), hipMemcpyHostToDevice, st));
     PF_HIP(hipEventRecord(dyn_done, st));
@@ -735,6 +738,12 @@ struct pf_batch {
     rows_total = r0;
     void* d = insts.get(n * sizeof(BatchInst));
     PF_HIP(hipMemcpy(d, recs.data(), n * sizeof(BatchInst), hipMemcpyHostToDevice));
+    if (!team_ok()) return;
+    const size_t sz = qsun_team_op_bytes();
+    std::vector<char> tr(n * sz);
+    for (int p = 0; p < n; ++p) qsun_team_op(ops[order[p]], tr.data() + p * sz);
+    d = trecs.get(n * sz);
+    PF_HIP(hipMemcpy(d, tr.data(), n * sz, hipMemcpyHostToDevice));
   }
   BatchArgs args() {
     BatchArgs A{};
@@ -864,6 +873,7 @@ struct pf_batch {
     drop_graph();
     if (cap) (void)hipStreamDestroy(cap);
     if (hdyn) (void)hipHostFree(hdyn);
+    if (hjobs) (void)hipHostFree(hjobs);
     if (dyn_done) (void)hipEventDestroy(dyn_done);
     insts.release();
     dyn.release();
@@ -871,8 +881,111 @@ struct pf_batch {
     coefs.release();
     kstate.release();
     bufs.release();
+    trecs.release();
+    tctl.release();
+    jobs.release();
+  }
+
+  // ---------------------------------------------------- the one-launch form
+  // Time of an application with orders k(p) (launch order, < 0: idle) on teams
+  // of 2^lt blocks: the longest job, or all jobs over all teams.
+  template <class F>
+  double team_us(int dtype, int lt, F&& k) const {
+    double sum = 0.0, most = 0.0;
+    for (int p = 0; p < n; ++p) {
+      const int K = k(p);
+      if (K < 0) continue;
+      const double us = (K + 1) * qsun_team_step_us(ops[order[p]], dtype, lt);
+      sum += us * s;
+      most = std::max(most, us);
+    }
+    return std::max(most, sum / (8 * (32 >> lt))) + 30.0;
+  }
+  // Blocks per column: every instance has to fit (also where the autotuner chose,
+  // which timed one arithmetic), and the estimate has to be below the per-step
+  // launches', which run in lockstep.
+  template <class F>
+  int team_choose(int dtype, F&& k) const {
+    if (team_forced || team == 0) return team;
+    int lo = 0;
+    while (team > 0 && (2 << lo) <= team) ++lo;
+    if (team > 0 && std::all_of(ops.begin(), ops.end(), [&](const pf_op* o) {
+          return qsun_team_fits(o, dtype, lo);
+        }))
+      return team;
+    int T = 0, kmax = -1;
+    double best = 1e300, elems = 0.0;
+    for (int lt = 0; lt < 6; ++lt) {
+      bool fit = true;
+      for (int p = 0; fit && p < n; ++p)
+        fit = qsun_team_ok(ops[p]) && qsun_team_fits(ops[p], dtype, lt);
+      if (!fit) continue;
+      const double us = team_us(dtype, lt, k);
+      if (us < best) {
+        best = us;
+        T = 1 << lt;
+      }
+    }
+    for (int p = 0; p < n; ++p) {
+      const int K = k(p);
+      kmax = std::max(kmax, K);
+      if (K >= 0) elems += (double)(K + 1) * ops[order[p]]->D * s;
+    }
+    // (elems / steps: rows of the mean step)
+    const double per = (kmax + 1) * qsun_per_step_us(elems / (kmax + 1), dtype);
+    return best < 0.9 * per ? T : 0;
+  }
+  bool team_ok() const {
+    for (const pf_op* o : ops)
+      if (!qsun_team_ok(o)) return false;
+    return true;
+  }
+  void team_ready() {
+    if (!tctl.p) tctl.get(team_ctl_bytes());
+    if (!jobs.p) jobs.get((size_t)n * s * sizeof(QsunJob));
+    if (!hjobs)
+      PF_HIP(hipHostMalloc(reinterpret_cast<void**>(&hjobs), (size_t)n * s * sizeof(QsunJob)));
+  }
+  // Launches the m jobs staged in hjobs, longest first.
+  void run_jobs(int m, int T, hipStream_t st) {
+    int lt = 0;
+    while ((2 << lt) <= T) ++lt;
+    std::sort(hjobs, hjobs + m, [&](const QsunJob& a, const QsunJob& b) {
+      const double ua = (a.K + 1) * qsun_team_step_us(ops[order[a.op]], a.dtype, lt);
+      const double ub = (b.K + 1) * qsun_team_step_us(ops[order[b.op]], b.dtype, lt);
+      return ua != ub ? ua > ub : a.X < b.X;
+    });
+    PF_HIP(hipMemcpyAsync(jobs.p, hjobs, m * sizeof(QsunJob), hipMemcpyHostToDevice, st));
+    PF_HIP(hipEventRecord(dyn_done, st));
+    dyn_pending = true;
+    qsun_team_batch(h, trecs.p, reinterpret_cast<const QsunJob*>(jobs.p), m,
+                    polytype, T, tctl.p, st);
   }
 };
+
+// Whether columns may finish in any order: no output overlaps another column's
+// input or output, nor its own input but for a column replaced in place.
+static bool batch_disjoint(const std::vector<QsunJob>& v, pf_op* const* ops,
+                           const std::vector<int>& order) {
+  struct Span {
+    const double *a, *e;
+    bool out;
+  };
+  std::vector<Span> sp;
+  for (const QsunJob& j : v) {
+    const int64_t D = ops[order[j.op]]->D;
+    if (j.X != j.Y) sp.push_back({j.X, j.X + D, false});
+    sp.push_back({j.Y, j.Y + D, true});
+  }
+  std::sort(sp.begin(), sp.end(), [](const Span& x, const Span& y) { return x.a < y.a; });
+  const double *ei = nullptr, *eo = nullptr;  // furthest ends of inputs and outputs so far
+  for (const Span& s : sp) {
+    if ((eo && s.a < eo) || (s.out && ei && s.a < ei)) return false;
+    const double*& e = s.out ? eo : ei;
+    if (!e || s.e > e) e = s.e;
+  }
+  return true;
+}
 
 extern "C" int pf_batch_create(pf_handle* h, int32_t n, pf_op* const* ops, int32_t ncols,
                                pf_batch** out) {
@@ -986,8 +1099,30 @@ extern "C" int pf_batch_filter(pf_batch* b, const int32_t* active, const int32_t
       mask |= dtypes[i] == PF_F64 ? kMaskF64 : kMaskF32;
     }
     if (kmax < 0) return;
-    b->upload_dyn(dy, st);
     char* base = reinterpret_cast<char*>(b->bufs.p);
+    const int T = b->team_ok() ? b->team_choose(mask & kMaskF64 ? PF_F64 : PF_F32,
+                                                [&](int p) { return dy[p].K; })
+                               : 0;
+    if (T) {
+      std::vector<QsunJob> v;
+      for (int i = 0; i < n; ++i) {
+        if (!active[i]) continue;
+        const int p = b->pos[i];
+        const int64_t D = b->ops[i]->D;
+        for (int c = 0; c < b->s; ++c)
+          v.push_back({X[i] + c * ldx[i], Y[i] + c * ldy[i],
+                       reinterpret_cast<const double*>(b->coefs.p) + b->coef_off[p],
+                       base + (b->row0[p] * b->s + c * D) * 16, p, dy[p].K, dtypes[i], 0});
+      }
+      if (batch_disjoint(v, b->ops.data(), b->order)) {
+        b->team_ready();
+        b->stage_ready();
+        std::copy(v.begin(), v.end(), b->hjobs);
+        b->run_jobs((int)v.size(), T, st);
+        return;
+      }
+    }
+    b->upload_dyn(dy, st);
     for (int i = 0; i < n; ++i) {
       if (!active[i]) continue;
       const int p = b->pos[i];
@@ -1014,32 +1149,46 @@ extern "C" int pf_batch_set_tuning(pf_batch* b, int32_t key, int32_t value) {
       case PF_BATCH_VEC:
         PF_REQUIRE(batch_vec_ok(b->s, value), "batch: vector width must divide ncols (1/2/4/8)");
         b->V = value;
+        b->team = 0, b->team_forced = false;  // (the knobs of the per-step forms select them)
         b->layout_blocks();
         break;
       case PF_BATCH_ROWS_PER_LANE:
         PF_REQUIRE(value >= 1 && value <= 64, "batch: 1 <= rows per lane <= 64");
         b->rpt = value;
+        b->team = 0, b->team_forced = false;
         b->layout_blocks();
         break;
       case PF_BATCH_XCD:
         PF_REQUIRE(value == 0 || value == 1, "batch: xcd 0/1");
         b->xcd = value;
+        b->team = 0, b->team_forced = false;
         b->drop_graph();
         break;
       case PF_BATCH_GRAIN_SHUFFLE:
         PF_REQUIRE(value == 0 || value == 1, "batch: grain shuffle 0/1");
         b->shfl = value;
+        b->team = 0, b->team_forced = false;
         b->drop_graph();
         break;
       case PF_BATCH_LDS_ROWS:
         PF_REQUIRE(value == 0 || value == 1, "batch: LDS rows 0/1");
         b->lds = value;
+        b->team = 0, b->team_forced = false;
         b->drop_graph();
         break;
       case PF_BATCH_ROW_VECTORS:
         PF_REQUIRE(value >= 0 && value <= 2, "batch: row vectors 0/1/2");
         b->rv = value;
+        b->team = 0, b->team_forced = false;
         b->layout_blocks();
+        break;
+      case PF_BATCH_TEAM:
+        PF_REQUIRE(value == -1 || value == 0 || value == 1 || value == 2 || value == 4 ||
+                       value == 8 || value == 16 || value == 32,
+                   "batch: blocks per column -1, 0, 1, 2, 4, 8, 16 or 32");
+        PF_REQUIRE(value <= 0 || b->team_ok(), "batch: an instance does not fit a team");
+        b->team = value;
+        b->team_forced = value > 0;
         break;
       default: throw Error{PF_ERR_INVALID, "batch: unknown tuning key"};
     }
@@ -1177,6 +1326,50 @@ extern "C" int pf_batch_autotune(pf_batch* b, int32_t dtype, int32_t nsteps, dou
       b->drop_graph();
       b->use_graph = g_us < s_us ? 1 : 0;
       best = std::min(g_us, s_us);
+    }
+    // the one-launch form, per step: two lengths of one application of all
+    // instances, from and to the work buffers (zero vectors)
+    b->team = 0;
+    b->team_forced = false;
+    if (b->team_ok()) {
+      b->team_ready();
+      DevBuf zero;
+      const int k1 = 16, k2 = 80;
+      double* c0 = reinterpret_cast<double*>(zero.get((k2 + 1) * sizeof(double)));
+      PF_HIP(hipMemsetAsync(c0, 0, (k2 + 1) * sizeof(double), st));
+      PF_HIP(hipMemsetAsync(b->bufs.p, 0, b->bufs.bytes, st));
+      double* io = reinterpret_cast<double*>(b->bufs.p) + 2 * b->rows_total * b->s;
+      for (int lt = 0; lt < 6; ++lt) {
+        if (!std::all_of(b->ops.begin(), b->ops.end(),
+                         [&](const pf_op* o) { return qsun_team_fits(o, dtype, lt); }))
+          continue;
+        double us[2] = {1e300, 1e300};
+        for (int round = 0; round < 3; ++round)
+          for (int w = 0; w < 2; ++w) {
+            b->stage_ready();
+            int m = 0;
+            for (int p = 0; p < n; ++p)
+              for (int c = 0; c < b->s; ++c) {
+                const int64_t D = b->ops[b->order[p]]->D, at = b->row0[p] * b->s + c * D;
+                b->hjobs[m++] = {io + at, io + b->rows_total * b->s + at, c0,
+                                 reinterpret_cast<char*>(b->bufs.p) + at * 16, p, w ? k2 : k1,
+                                 dtype, 0};
+              }
+            PF_HIP(hipEventRecord(e0, st));
+            b->run_jobs(m, 1 << lt, st);
+            PF_HIP(hipEventRecord(e1, st));
+            PF_HIP(hipEventSynchronize(e1));
+            float ms = 0.f;
+            PF_HIP(hipEventElapsedTime(&ms, e0, e1));
+            us[w] = std::min(us[w], 1e3 * ms);
+          }
+        const double t = (us[1] - us[0]) / (k2 - k1);
+        if (t < 0.99 * best) {
+          best = t;
+          b->team = 1 << lt;
+        }
+      }
+      zero.release();
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);

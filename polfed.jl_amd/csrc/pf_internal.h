@@ -261,6 +261,32 @@ size_t team_kpm_bytes(const pf_op* op, int dtype, int N, int ncols, int T);
 void team_kpm(pf_op* op, int dtype, int N, const double* X, int64_t ldx, int ncols,
               const double* colscale, double* mu, int T, void* work, hipStream_t st);
 
+size_t team_ctl_bytes();
+void team_begin(void* ctl, double* cdev, const double* coeffs, int order, hipStream_t st);
+
+// Quantum-Sun filters in one launch (qteam.hip): a job is one column of one
+// instance; work holds two vectors of its rows.
+struct QsunJob {
+  const double* X;
+  double* Y;
+  const double* coefs;
+  char* work;
+  int32_t op, K, dtype, pad;
+};
+size_t qsun_team_op_bytes();
+void qsun_team_op(const pf_op* op, void* rec);
+bool qsun_team_ok(const pf_op* op);
+bool qsun_team_fits(const pf_op* op, int dtype, int lt);
+double qsun_team_step_us(const pf_op* op, int dtype, int lt);
+double qsun_per_step_us(double elems, int dtype);
+void qsun_team_batch(const pf_handle* h, const void* recs,
+                     const QsunJob* jobs, int njobs, int polytype, int T, void* ctl,
+                     hipStream_t st);
+size_t qsun_team_work_bytes(const pf_op* op, int dtype, int order, int ncols, int T);
+void qsun_team_filter(pf_op* op, int dtype, int polytype, const double* coeffs, int order,
+                      const double* X, int64_t ldx, double* Y, int64_t ldy, int ncols, int T,
+                      void* work, hipStream_t st);
+
 // Looks up this device's address of pf_filter_noalloc's scratch array once per
 // device (ops.hip); called by pf_create with the device current.
 void noalloc_scratch_init(int device);

@@ -18,6 +18,16 @@ namespace pf {
 constexpr int kMaxDg = 1 << kMaxGrain;
 constexpr int kMaxLocPad = 32;  // outer spins padded to whole gather batches
 
+// The recurrence's alpha_k and beta_k.
+__device__ __forceinline__ void poly_ab_dev(int type, int k, double& alpha, double& beta_k) {
+  switch (type) {
+    case PF_LEGENDRE: alpha = (2.0 * k + 1) / (k + 1); beta_k = -(double)k / (k + 1); break;
+    case PF_HERMITE: alpha = 2.0; beta_k = -2.0 * k; break;
+    case PF_TAYLOR: alpha = 1.0; beta_k = 0.0; break;
+    default: alpha = 2.0; beta_k = -1.0; break;  // Chebyshev
+  }
+}
+
 // Per-block constants of one Quantum-Sun operator in one step.
 struct QsunRow {
   const char* b2;        // base of the b2 block (bytes), uniform

@@ -158,4 +158,131 @@ __device__ __forceinline__ bool team_wait(TeamCtl* c, TeamPlace& me) {
   });
 }
 
+constexpr int kTeamThreads = 1024;
+constexpr int kTeamWaves = kTeamThreads / 64;
+
+// A value that is the same in all lanes, as a scalar.
+__device__ __forceinline__ uint32_t uni(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+
+
+// Uniform read-only data through the scalar cache.
+template <typename S>
+__device__ __forceinline__ S cload(const S* p) {
+  typedef const __attribute__((address_space(4))) S* cp;
+  return *(cp)(uintptr_t)p;
+}
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kAgent = 16;  // buffer instruction cache policy: sc1
+
+// Loads of 4, 8 or 16 bytes at voff + soff bytes, at agent scope.  (Stores
+// take the default policy: they pass the CU's L1 and stay in the L2, where a
+// store at agent scope is written through to memory, at half the rate.)
+template <typename V>
+__device__ __forceinline__ V bload(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+  if constexpr (sizeof(V) == 16)
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kAgent));
+  else if constexpr (sizeof(V) == 8)
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, kAgent));
+  else
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, kAgent));
+}
+template <typename V>
+__device__ __forceinline__ void bstore(V v, __amdgpu_buffer_rsrc_t r, uint32_t voff,
+                                       uint32_t soff) {
+  if constexpr (sizeof(V) == 16)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, 0);
+  else if constexpr (sizeof(V) == 4)
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, soff, 0);
+  else
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, voff, soff, 0);
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, bytes, 0x00027000);
+}
+
+// LDS at a byte offset of the dynamic block.
+extern __shared__ __align__(16) char team_lds[];
+template <typename T>
+__device__ __forceinline__ T lread(uint32_t off) {
+  typedef const __attribute__((address_space(3))) T* lp;
+  typedef const __attribute__((address_space(3))) char* lc;
+  return *(lp)((lc)team_lds + off);
+}
+template <typename T>
+__device__ __forceinline__ void lwrite(uint32_t off, T v) {
+  typedef __attribute__((address_space(3))) T* lp;
+  typedef __attribute__((address_space(3))) char* lc;
+  *(lp)((lc)team_lds + off) = v;
+}
+
+// What the blocks of a team share about the job in hand.
+struct TeamShared {
+  uint32_t idx, n, bar, slot, ok, job, seg, pad[9];
+  double red[2 * kTeamWaves];  // the waves' dots of a step
+};
+
+// Both halves of the barrier around `between` (this block's own LDS update).
+template <class F>
+__device__ __forceinline__ bool team_step_end(TeamCtl* ctl, TeamShared& sh, TeamPlace& me,
+                                              bool read_job, F&& between) {
+  team_drain();
+  __syncthreads();
+  if (threadIdx.x < 64) team_arrive(me);
+  between();
+  if (threadIdx.x < 64) {
+    const bool ok = team_wait(ctl, me);
+    if (threadIdx.x == 0) {
+      if (ok && read_job && me.n > 1) sh.job = team_load(&me.bar->job);
+      sh.ok = ok;
+      sh.seg = 0;
+    }
+  }
+  __syncthreads();
+  return uni(sh.ok) != 0;
+}
+
+// Joins a team (wave 0 polls the barrier with all its lanes, so every thread gets
+// the place); false: none, or the abort flag.  `between` runs before the team's
+// first barrier.  sh.slot: the team's number among all teams.
+template <class F>
+__device__ __forceinline__ bool team_enter(TeamCtl* ctl, uint32_t expect, uint32_t want,
+                                           TeamShared& sh, TeamPlace& me, F&& between) {
+  if (threadIdx.x == 0) {
+    sh.ok = team_join(ctl, expect, want, me);
+    if (sh.ok) {
+      sh.idx = me.idx;
+      sh.n = me.n;
+      sh.bar = (uint32_t)(me.bar - ctl->bar);
+      if (me.idx == 0) {
+        sh.slot = team_add(&ctl->slots, 1u);
+        if (me.n > 1) team_store(&me.bar->slot, sh.slot);
+      }
+    }
+  }
+  __syncthreads();
+  if (!uni(sh.ok)) return false;
+  me.idx = uni(sh.idx);
+  me.n = uni(sh.n);
+  me.bar = &ctl->bar[uni(sh.bar)];
+  me.passed = 0;
+  between();
+  if (!team_step_end(ctl, sh, me, false, [] {})) return false;
+  if (threadIdx.x == 0 && me.n > 1) sh.slot = team_load(&me.bar->slot);
+  __syncthreads();
+  return true;
+}
+
+// Next column of this team, or >= ncols when none is left; false: abort.
+__device__ __forceinline__ bool team_next(TeamCtl* ctl, TeamShared& sh, TeamPlace& me) {
+  __syncthreads();  // the last job's readers of `sh` and of LDS are done
+  if (threadIdx.x == 0 && me.idx == 0) {
+    sh.job = team_add(&ctl->next, 1u);
+    if (me.n > 1) team_store(&me.bar->job, sh.job);
+  }
+  return team_step_end(ctl, sh, me, true, [] {});
+}
+
 }  // namespace pf

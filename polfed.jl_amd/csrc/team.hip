@@ -42,8 +42,6 @@
 
 namespace pf {
 
-constexpr int kTeamThreads = 1024;
-constexpr int kTeamWaves = kTeamThreads / 64;
 
 // kGrp consecutive rows of one segment, two per lane.
 constexpr uint32_t kGrp = 128;
@@ -121,60 +119,12 @@ struct TeamArgs {
 constexpr uint32_t tab_rows(int NC) { return NC == 0 ? 2050u : 1048u; }
 constexpr int kTeamUnits = 32;  // streaming work lists (dealt to the blocks of a team)
 
-// Uniform read-only data through the scalar cache.
-template <typename S>
-__device__ __forceinline__ S cload(const S* p) {
-  typedef const __attribute__((address_space(4))) S* cp;
-  return *(cp)(uintptr_t)p;
-}
 __device__ __forceinline__ TeamGrp cload_grp(const TeamGrp* p) {
   typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
   static_assert(sizeof(TeamGrp) == sizeof(u32x8));
   return __builtin_bit_cast(TeamGrp, cload(reinterpret_cast<const u32x8*>(p)));
 }
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-constexpr int kAgent = 16;  // buffer instruction cache policy: sc1
-
-// Loads of V = T or a pair of T at voff + soff bytes, at agent scope.  (Stores
-// take the default policy: they pass the CU's L1 and stay in the L2, where a
-// store at agent scope is written through to memory, at half the rate.)
-template <typename V>
-__device__ __forceinline__ V bload(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  if constexpr (sizeof(V) == 16)
-    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kAgent));
-  else if constexpr (sizeof(V) == 8)
-    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, kAgent));
-  else
-    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, kAgent));
-}
-template <typename V>
-__device__ __forceinline__ void bstore(V v, __amdgpu_buffer_rsrc_t r, uint32_t voff,
-                                       uint32_t soff) {
-  if constexpr (sizeof(V) == 16)
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, 0);
-  else
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, voff, soff, 0);
-}
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(p, 0, bytes, 0x00027000);
-}
-
-// LDS at a byte offset of the dynamic block.
-extern __shared__ __align__(16) char team_lds[];
-template <typename T>
-__device__ __forceinline__ T lread(uint32_t off) {
-  typedef const __attribute__((address_space(3))) T* lp;
-  typedef const __attribute__((address_space(3))) char* lc;
-  return *(lp)((lc)team_lds + off);
-}
-template <typename T>
-__device__ __forceinline__ void lwrite(uint32_t off, T v) {
-  typedef __attribute__((address_space(3))) T* lp;
-  typedef __attribute__((address_space(3))) char* lc;
-  *(lp)((lc)team_lds + off) = v;
-}
 
 __device__ __forceinline__ void team_ab(int type, int k, double& alpha, double& beta_k) {
   switch (type) {
@@ -370,17 +320,6 @@ __device__ __forceinline__ TeamCoef<T> team_coef(const TeamArgs& A, int j) {
   return {(T)ck, (T)alpha, (T)beta};
 }
 
-// A value that is the same in all lanes, as a scalar.
-__device__ __forceinline__ uint32_t uni(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
-}
-
-// What the blocks of a team share about the job in hand.
-struct TeamShared {
-  uint32_t idx, n, bar, slot, ok, job, seg, pad[9];
-  double red[2 * kTeamWaves];  // the waves' dots of a step
-};
-
 // KPM dots of one step.  FP64: <T_{j-1}, T_{j-1}> and <T_j, T_{j-1}>, from which
 // mu_{2j-2} and mu_{2j-1} follow (2 T_m T_n = T_{m+n} + T_{m-n}): half the steps of
 // the direct form.  FP32: <x, x> and <x, T_j>, because there the identity's
@@ -418,36 +357,6 @@ __device__ __forceinline__ void team_dots_out(const TeamArgs& A, const TeamShare
     for (int i = 0; i < kTeamWaves; ++i) t += sh.red[2 * i + w];
     A.dots[((int64_t)(2 * (j - 1) + (int)w) * A.ncols + col) * kTeamUnits + idx] = t;
   }
-}
-
-// Both halves of the barrier around `between` (this block's own LDS update).
-template <class F>
-__device__ __forceinline__ bool team_step_end(const TeamArgs& A, TeamShared& sh, TeamPlace& me,
-                                              bool read_job, F&& between) {
-  team_drain();
-  __syncthreads();
-  if (threadIdx.x < 64) team_arrive(me);
-  between();
-  if (threadIdx.x < 64) {
-    const bool ok = team_wait(A.ctl, me);
-    if (threadIdx.x == 0) {
-      if (ok && read_job && me.n > 1) sh.job = team_load(&me.bar->job);
-      sh.ok = ok;
-      sh.seg = 0;
-    }
-  }
-  __syncthreads();
-  return uni(sh.ok) != 0;
-}
-
-// Next column of this team, or >= ncols when none is left; false: abort.
-__device__ __forceinline__ bool team_next(const TeamArgs& A, TeamShared& sh, TeamPlace& me) {
-  __syncthreads();  // the last job's readers of `sh` and of LDS are done
-  if (threadIdx.x == 0 && me.idx == 0) {
-    sh.job = team_add(&A.ctl->next, 1u);
-    if (me.n > 1) team_store(&me.bar->job, sh.job);
-  }
-  return team_step_end(A, sh, me, true, [] {});
 }
 
 // The streaming form of one column (any team size, any D).
@@ -538,7 +447,7 @@ __device__ bool stream_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me, 
       dots.park(sh);
       dots = TeamDots{};
     }
-    if (j < steps && !team_step_end(A, sh, me, false, [&] {
+    if (j < steps && !team_step_end(A.ctl, sh, me, false, [&] {
           if (KPM && !first) team_dots_out(A, sh, j, col, me.idx);
         }))
       return false;
@@ -649,7 +558,7 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
     int zero;  // (opaque: the R conditions are not hoisted into saved masks)
     asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
     left = mine + zero;
-    if (!team_step_end(A, sh, me, false, [&] {
+    if (!team_step_end(A.ctl, sh, me, false, [&] {
           // p holds the new vector, LDS still the one before: exchange them
 #pragma unroll
           for (int r = 0; r < R; ++r)
@@ -784,6 +693,8 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
 template <typename T, int NQ, int NC, bool UNI, bool KPM, int R>
 __global__ __launch_bounds__(kTeamThreads) void chain_team_kernel(const TeamArgs A) {
   TeamShared& sh = *reinterpret_cast<TeamShared*>(team_lds + A.rows_lds);
+  // (team_enter in line: as a call, even inlined, the R = 4 form spills 34 registers
+  // instead of 18 and a step at L = 20 takes 4 % longer)
   TeamPlace me{};
   if (threadIdx.x == 0) {
     sh.ok = team_join(A.ctl, (uint32_t)A.expect, (uint32_t)A.T, me);
@@ -821,14 +732,14 @@ __global__ __launch_bounds__(kTeamThreads) void chain_team_kernel(const TeamArgs
         lwrite<uint32_t>(t, 0u);
     }
   }
-  if (!team_step_end(A, sh, me, false, [] {})) return;
+  if (!team_step_end(A.ctl, sh, me, false, [] {})) return;
   if (threadIdx.x == 0 && me.n > 1) sh.slot = team_load(&me.bar->slot);
   __syncthreads();
   const uint32_t slot = uni(sh.slot);
   if (slot >= (uint32_t)A.nslots) return;  // (uniform over the team)
   char* work = A.work + (int64_t)slot * A.slot_bytes;
   while (true) {
-    if (!team_next(A, sh, me)) return;
+    if (!team_next(A.ctl, sh, me)) return;
     const uint32_t col = uni(sh.job);
     if (col >= (uint32_t)A.ncols) return;
     bool ok;
@@ -1314,7 +1225,9 @@ static double team_step_us(const TeamTables* t, int dtype, int ncols, int lt) {
 // The per-step kernels: launch-bound below 5 us, then at the rate of their
 // algorithmic bytes (2.6 TB/s; half that when the blocks exceed the 256 MB
 // Infinity Cache).
-static double per_step_us(int64_t D, int dtype, int ncols) {
+static double per_step_us(const pf_op* op, int dtype, int ncols) {
+  const int64_t D = op->D;
+  if (op->kind == kQsun) return qsun_per_step_us((double)D * ncols, dtype);
   const double mb = 4e-6 * (double)D * ncols * (dtype == PF_F64 ? 8 : 4);
   return std::max(5.0, mb / (mb > 512 ? 1.4 : 2.6));
 }
@@ -1324,9 +1237,19 @@ int team_kpm_steps(int dtype, int N);
 // Blocks per column of the fastest team form, and its time.
 int team_best(const pf_op* op, int dtype, int ncols, double* us) {
   const TeamTables* t = op->team;
-  if (!t) return 0;
   int best = 0;
   *us = 1e300;
+  if (op->kind == kQsun && qsun_team_ok(op))
+    for (int lt = 0; lt < 6; ++lt) {
+      if (!qsun_team_fits(op, dtype, lt)) continue;
+      const int teams = 8 * (32 >> lt);
+      const double x = (ncols + teams - 1) / teams * qsun_team_step_us(op, dtype, lt);
+      if (x < *us) {
+        *us = x;
+        best = 1 << lt;
+      }
+    }
+  if (!t) return best;
   for (int lt = 0; lt < 6; ++lt) {
     if ((t->NC == 0) != (lt == 0)) continue;
     const double x = team_step_us(t, dtype, ncols, lt);
@@ -1346,8 +1269,9 @@ constexpr int kTeamMinOrder = 8;
 static int team_choose(const pf_op* op, int dtype, int order, int ncols, int gain) {
   const TeamTables* t = op->team;
   const TuneCfg& f = op->force;
-  if (!t || order < 1 || f.team == 0) return 0;
-  if (f.team > 0) return t->NC == 0 ? 1 : f.team;
+  const bool qsun = op->kind == kQsun && qsun_team_ok(op);
+  if ((!t && !qsun) || order < 1 || f.team == 0) return 0;
+  if (f.team > 0) return t && t->NC == 0 ? 1 : f.team;
   // forced launch knobs are those of the per-step kernels
   if (f.V || f.xcd >= 0 || f.nt >= 0 || f.pb >= 0 || f.wide >= 0 || f.occ >= 0 || f.part >= 0)
     return 0;
@@ -1358,7 +1282,7 @@ static int team_choose(const pf_op* op, int dtype, int order, int ncols, int gai
     return it->second.team;
   double us;
   const int T = team_best(op, dtype, ncols, &us);
-  return us < 0.95 * gain * per_step_us(op->D, dtype, ncols) ? T : 0;
+  return us < 0.95 * gain * per_step_us(op, dtype, ncols) ? T : 0;
 }
 
 int team_plan(const pf_op* op, int dtype, int polytype, int order, const double* X, int64_t ldx,
@@ -1376,12 +1300,27 @@ int team_plan(const pf_op* op, int dtype, int polytype, int order, const double*
 // 16); 16 probes, L = 22: 9.1 -> 2.9 ms at N = 60 (streamed); FP32, the same steps:
 // L = 20 8.0 -> 5.3 ms, L = 18 2.9 -> 1.5 ms (team of 8).
 int team_kpm_plan(const pf_op* op, int dtype, int N, int ncols) {
+  if (!op->team) return 0;
   return team_choose(op, dtype, team_kpm_steps(dtype, N), ncols, dtype == PF_F64 ? 2 : 1);
 }
 
 static size_t team_align(size_t n) { return (n + 255) & ~(size_t)255; }
+size_t team_ctl_bytes() { return team_align(sizeof(TeamCtl)); }
+
+// Clears the control words and copies order + 1 coefficients.
+void team_begin(void* ctl, double* cdev, const double* coeffs, int order, hipStream_t st) {
+  for (int at = 0; at == 0 || at <= order; at += kCoefChunk) {
+    TeamCoefs c;
+    const int n = std::max(0, std::min(kCoefChunk, order + 1 - at));
+    if (n) std::memcpy(c.c, coeffs + at, n * sizeof(double));
+    hipLaunchKernelGGL(team_begin_kernel, dim3(1), dim3(1024), 0, st,
+                       at ? nullptr : static_cast<TeamCtl*>(ctl), cdev, at, n, c);
+    PF_HIP(hipGetLastError());
+  }
+}
 
 size_t team_work_bytes(const pf_op* op, int dtype, int order, int ncols, int T) {
+  if (op->kind == kQsun) return qsun_team_work_bytes(op, dtype, order, ncols, T);
   const size_t vec = (size_t)op->team->elems * (dtype == PF_F64 ? 8 : 4);
   return team_align(sizeof(TeamCtl)) + team_align((size_t)(order + 1) * 8) +
          std::min(ncols, 8 * (32 / T)) * 3 * vec;
@@ -1487,16 +1426,11 @@ static void team_run(pf_op* op, int dtype, TeamArgs A, int T, void* work, size_t
 void team_filter(pf_op* op, int dtype, int polytype, const double* coeffs, int order,
                  const double* X, int64_t ldx, double* Y, int64_t ldy, int ncols, int T,
                  void* work, hipStream_t st) {
+  if (op->kind == kQsun)
+    return qsun_team_filter(op, dtype, polytype, coeffs, order, X, ldx, Y, ldy, ncols, T, work, st);
   TeamCtl* ctl = (TeamCtl*)work;
-  double* cdev = (double*)((char*)work + team_align(sizeof(TeamCtl)));
-  for (int at = 0; at <= order; at += kCoefChunk) {
-    TeamCoefs c;
-    const int n = std::min(kCoefChunk, order + 1 - at);
-    std::memcpy(c.c, coeffs + at, n * sizeof(double));
-    hipLaunchKernelGGL(team_begin_kernel, dim3(1), dim3(1024), 0, st, at ? nullptr : ctl, cdev, at,
-                       n, c);
-    PF_HIP(hipGetLastError());
-  }
+  double* cdev = (double*)((char*)work + team_ctl_bytes());
+  team_begin(ctl, cdev, coeffs, order, st);
   TeamArgs A{};
   A.order = order;
   A.polytype = polytype;
@@ -1560,8 +1494,7 @@ void team_kpm(pf_op* op, int dtype, int N, const double* X, int64_t ldx, int nco
   double* dots = (double*)((char*)work + team_work_bytes(op, dtype, 0, ncols, T));
   const int64_t n = (int64_t)2 * steps * ncols * kTeamUnits;
   double* sums = (double*)((char*)dots + team_align(n * 8));
-  TeamCoefs none{};
-  hipLaunchKernelGGL(team_begin_kernel, dim3(1), dim3(1024), 0, st, ctl, nullptr, 0, 0, none);
+  team_begin(ctl, nullptr, nullptr, -1, st);
   hipLaunchKernelGGL(team_zero_kernel, dim3(512), dim3(256), 0, st, dots, n);
   PF_HIP(hipGetLastError());
   TeamArgs A{};
