@@ -225,6 +225,97 @@ __global__ __launch_bounds__(256) void chain_step_kernel(PF_CHAIN_ARGS) {
   chain_step_body<T, V, GM, TBL, NBW>(PF_CHAIN_PASS);
 }
 
+constexpr int kCols = 4, kColsBatch = 4;  // columns per lane, bonds at a time
+
+// One step on column-major blocks, C columns per lane (the last group fewer): the
+// ranks of a row's neighbours, two thirds of the instructions with one column per
+// lane, are found once for C columns.  Then the gathers bound it (1.0 GB through
+// the vector caches at L = 22, 16 FP64 columns; eight columns, or more bonds at a
+// time, take the same).  One application on 16 columns at L = 22: FP64 184 -> 126
+// us, FP32 149 -> 70; 8 columns at L = 20, J1-J2: 37 -> 31.
+template <typename T, int C, bool TBL>
+__global__ __launch_bounds__(256) void chain_cols_kernel(
+    const ChainParams P, const uint32_t* __restrict__ states, const uint32_t* __restrict__ binom,
+    const uint4* __restrict__ rtab, const int rtab_vec, const double* __restrict__ diag,
+    const Affine af, const int flags, const T cx, const T ch, const T cb, const T* X,
+    const T* __restrict__ B2, const T* B3, T* OUT, const int64_t ld, const int ncols,
+    const int64_t ngroups) {
+  constexpr int NB = kColsBatch;
+  extern __shared__ uint4 tab_lds[];
+  __shared__ uint32_t sM[kMaxBonds];
+  __shared__ T sW[kMaxBonds];
+  RankCtx R{};
+  R.M = sM;
+  if constexpr (TBL) {
+    for (int i = threadIdx.x; i < rtab_vec; i += blockDim.x) tab_lds[i] = rtab[i];
+    R.TA = reinterpret_cast<const uint16_t*>(tab_lds);
+    R.TB = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(tab_lds) +
+                                             (2u << P.tsplit));
+    R.maskA = (1u << P.tsplit) - 1u;
+    R.m = P.tsplit;
+  } else {
+    __shared__ uint32_t sC[32 * kRankT];
+    for (int i = threadIdx.x; i < 32 * kRankT; i += blockDim.x) sC[i] = binom[i];
+    R.C = sC;
+  }
+  const int nbp = (P.nb + NB - 1) / NB * NB;  // padded with zero bonds
+  for (int i = threadIdx.x; i < nbp; i += blockDim.x) {
+    const bool real = i < P.nb;
+    sW[i] = real ? (T)(P.bval[i] * af.scale) : (T)0;
+    sM[i] = real ? (1u << P.lo[i]) | (1u << P.hi[i]) : 0u;
+  }
+  __syncthreads();
+
+  const int c0 = blockIdx.y * C, nc = ncols - c0 < C ? ncols - c0 : C;  // uniform
+  const T* b2[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) b2[c] = B2 + (int64_t)(c0 + (c < nc ? c : 0)) * ld;
+  const int64_t p = xcd_block(blockIdx.x, gridDim.x);
+  const int64_t g_end = (p + 1) * ngroups / gridDim.x;
+  for (int64_t grp = p * ngroups / gridDim.x; grp < g_end; ++grp) {
+    const int64_t row = grp * 256 + threadIdx.x;
+    if (row >= P.D) continue;
+    const uint32_t r32 = (uint32_t)row, st = states[row];
+    T tot[C], own[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      tot[c] = (T)0;
+      own[c] = b2[c][row];
+    }
+    for (int b0 = 0; b0 < nbp; b0 += NB) {
+      uint32_t rk[NB];
+      bond_ranks<1, NB, TBL>(R, b0, st, r32, 0, rk);
+      T x[NB][C];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) x[j][c] = (T)0;
+        if (rk[j] != r32) {
+#pragma unroll
+          for (int c = 0; c < C; ++c) x[j][c] = b2[c][rk[j]];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const T w = sW[b0 + j];
+#pragma unroll
+        for (int c = 0; c < C; ++c) tot[c] += w * x[j][c];
+      }
+    }
+    const T d = (T)((diag[row] - af.shift) * af.scale);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (c >= nc) break;
+      const int64_t o = row + (int64_t)(c0 + c) * ld;
+      T v = (T)0;
+      if (flags & kHasX) v = cx * X[o];
+      v += ch * (d * own[c] + tot[c]);
+      if (flags & kHasB3) v += cb * B3[o];
+      OUT[o] = v;
+    }
+  }
+}
+
 // The same step held to 8 waves per SIMD (at most 64 VGPRs): more rows in
 // flight per CU to hide the neighbour-gather latency, at the price of fewer
 // gathers in flight per wave.
@@ -398,6 +489,24 @@ static void launch_typed(pf_op* op, int flags, const Layout& lay, int ncols_grid
   const T* Pt = reinterpret_cast<const T*>(P);
   if (op->kind == kChain) {
     const bool tbl = op->chain.tsplit > 0 && op->rtab;
+    if constexpr (V == 1) {
+      // Column-major blocks with enough work for four blocks of rows and columns per
+      // CU (L = 20, two columns, 722 blocks: 9.7 us with a column per lane, 10.9 so;
+      // L = 18, 32 columns, 1520 blocks: 26.8 and 18.3).
+      const int cb4 = (ncols_grid + kCols - 1) / kCols;
+      if (lay.rs == 1 && ncols_grid > 1 && ngroups * cb4 >= 4 * op->h->prop.multiProcessorCount &&
+          (flags & kHasH) && !(flags & (kOutCM | kDot))) {
+        const dim3 g((unsigned)gx, (unsigned)cb4);
+        auto* k = tbl ? chain_cols_kernel<T, kCols, true> : chain_cols_kernel<T, kCols, false>;
+        hipLaunchKernelGGL(k, g, block, tbl ? op->rtab_bytes : 0, st, op->chain, op->states,
+                           op->binom, reinterpret_cast<const uint4*>(op->rtab),
+                           (int)(op->rtab_bytes / 16), op->diag, af, flags, (T)cx, (T)ch, (T)cb,
+                           Xt, B2t, B3t, reinterpret_cast<T*>(out), lay.cstride, ncols_grid,
+                           ngroups);
+        PF_HIP(hipGetLastError());
+        return;
+      }
+    }
     // drivers run in the partition order when it is built; the hooks never do
     const bool part = (flags & kRowPart) && op->pstates;
     const uint32_t* sts = part ? op->pstates : op->states;
