@@ -45,6 +45,7 @@ extern "C" int pf_destroy(pf_handle* h) {
   h->partials.release();
   h->small.release();
   h->vecs.release();
+  if (h->pinned) (void)hipHostFree(h->pinned);
   delete h;
   return PF_OK;
 }

@@ -26,9 +26,15 @@ __device__ __forceinline__ d4 mfma16x16x4(double a, double b, d4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-constexpr int kGramRowBlocks = 128;  // row partitions of the Gram reduction
+// row partitions of the Gram reduction: two blocks per CU and 128 columns of a wide A
+// (614 MB: 170 us with 128, 161 so), half of it for one tile of columns, whose
+// partials one block adds up
+constexpr int kGramRowBlocks = 256, kGramRowBlocks1 = 128;
 constexpr int kMaxN = 64;            // widest B block of the Gram/update kernels
 
+// WS: A has at most 16 columns; the four waves take every fourth slab each and add
+// their tiles in LDS (184756 x 8: 28.4 us with three waves idle, 10.1 us so).
+//
 // Gram partials: part[(rb * m + i) * n + j] = sum over rb's slabs of A[:, i] B[:, j].
 // Grid: (kGramRowBlocks, ceil(m/(64*AT))); block: 4 waves, wave w owns the AT
 // tiles of 16 A columns from i0 = 64*AT*blockIdx.y + 16*AT*w and all n columns
@@ -37,12 +43,12 @@ constexpr int kMaxN = 64;            // widest B block of the Gram/update kernel
 // a time with every load issued before the first MFMA.  Lanes past m or n
 // read a clamped column (their results are not stored); only the rows past D
 // of the last, partial slab are zeroed.
-template <int NT, int AT>
+template <int NT, int AT, bool WS = false>
 __global__ __launch_bounds__(256) void gram_kernel(const double* __restrict__ A, int64_t lda, int m,
                                                    const double* __restrict__ B, int64_t ldb, int n,
                                                    int64_t D, double* __restrict__ part) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int i0 = (blockIdx.y * 64 + w * 16) * AT;
+  const int i0 = WS ? 0 : (blockIdx.y * 64 + w * 16) * AT;
   const int li = lane & 15, kq = lane >> 4;
   const double* pa[AT];
 #pragma unroll
@@ -81,8 +87,9 @@ __global__ __launch_bounds__(256) void gram_kernel(const double* __restrict__ A,
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[a][t] = mfma16x16x4(av[a][q], bv[t][q], acc[a][t]);
   };
-  const int64_t gx = gridDim.x, nfull = D / 16;
-  int64_t sl = blockIdx.x;
+  const int64_t gx = WS ? 4 * gridDim.x : gridDim.x, nfull = D / 16;
+  const int64_t first = WS ? 4 * blockIdx.x + w : blockIdx.x;
+  int64_t sl = first;
   for (; sl + gx < nfull; sl += 2 * gx) {
     double av0[AT][4], bv0[NT][4], av1[AT][4], bv1[NT][4];
     load(sl * 16 + 4 * kq, false, av0, bv0);
@@ -95,10 +102,23 @@ __global__ __launch_bounds__(256) void gram_kernel(const double* __restrict__ A,
     load(sl * 16 + 4 * kq, false, av, bv);
     fma(av, bv);
   }
-  if (D % 16 != 0 && blockIdx.x == nfull % gx) {  // the partial last slab
+  if (D % 16 != 0 && first == nfull % gx) {  // the partial last slab
     double av[AT][4], bv[NT][4];
     load(nfull * 16 + 4 * kq, true, av, bv);
     fma(av, bv);
+  }
+  if constexpr (WS) {
+    __shared__ d4 sum[3][NT][64];
+    if (w > 0) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) sum[w - 1][t][lane] = acc[0][t];
+    }
+    __syncthreads();
+    if (w > 0) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) acc[0][t] += sum[k][t][lane];
   }
   // D-fragment: row (A column) i0 + 16a + kq + 4*v, column (B column) 16*t + li
   double* out = part + (int64_t)blockIdx.x * m * n;
@@ -116,27 +136,35 @@ __global__ __launch_bounds__(256) void gram_kernel(const double* __restrict__ A,
 }
 
 // G[i*gsi + j*gsj] = sum_rb part[(rb*m + i)*n + j]  (fixed order:
-// deterministic).  The partials are loaded 16 at a time before they are added
-// in order, so one memory round trip serves 16 terms.
-__global__ void gram_reduce_kernel(const double* __restrict__ part, int nrb, int m, int n,
-                                   double* __restrict__ G, int64_t gsi, int64_t gsj) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)m * n) return;
-  const int i = (int)(idx / n), j = (int)(idx % n);
+// deterministic).  Eight lanes per entry take every eighth partial, 16 loads at a
+// time, and add their sums pairwise (416 x 8 entries: 8.7 us for 128 partials with a
+// lane per entry, 5.1 us so for 256).
+__global__ __launch_bounds__(256) void gram_reduce_kernel(const double* __restrict__ part, int nrb,
+                                                          int m, int n, double* __restrict__ G,
+                                                          int64_t gsi, int64_t gsj) {
+  // lanes of consecutive entries, so that each load is one line
+  const int e = threadIdx.x & 31, k = threadIdx.x >> 5;
+  const int64_t idx = (int64_t)blockIdx.x * 32 + e;
   const int64_t stride = (int64_t)m * n;
-  const double* p = part + (int64_t)i * n + j;
+  __shared__ double red[8][32];
   constexpr int U = 16;
   double t = 0.0;
-  int rb = 0;
-  for (; rb + U <= nrb; rb += U, p += U * stride) {
-    double v[U];
+  if (idx < stride) {
+    for (int rb = k; rb < nrb; rb += 8 * U) {
+      double v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = p[u * stride];
+      for (int u = 0; u < U; ++u) v[u] = rb + 8 * u < nrb ? part[(rb + 8 * u) * stride + idx] : 0.0;
 #pragma unroll
-    for (int u = 0; u < U; ++u) t += v[u];
+      for (int u = 0; u < U; ++u) t += v[u];
+    }
   }
-  for (; rb < nrb; ++rb, p += stride) t += *p;
-  G[i * gsi + j * gsj] = t;
+  red[k][e] = t;
+  __syncthreads();
+  if (k == 0 && idx < stride) {
+    const double a = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
+    const double b = (red[4][e] + red[5][e]) + (red[6][e] + red[7][e]);
+    G[(idx / n) * gsi + (idx % n) * gsj] = a + b;
+  }
 }
 
 // B = beta*B + alpha*A*G.  Block: 4 waves, 64 rows (wave w: rows r0+16w..+15),
@@ -207,22 +235,128 @@ __global__ __launch_bounds__(256) void update_kernel(const double* __restrict__ 
   }
 }
 
-// W[r, :] = W[r, :] * M for an n x n matrix M (column-major), one row per thread.
-__global__ __launch_bounds__(256) void rotate_kernel(double* __restrict__ W, int64_t ldw, int64_t D,
-                                                     int n, const double* __restrict__ M) {
-  __shared__ double sM[kMaxN * kMaxN];
-  for (int i = threadIdx.x; i < n * n; i += blockDim.x) sM[i] = M[i];
+// dst[r, :] = src[r, :] * M for an n x n matrix M (column-major), one row per
+// thread held in N >= n registers (an array of run-time length went through
+// scratch memory: 184756 x 8 took 21.7 us, 6.5 us so); TRI: M is upper triangular.
+// src and dst may be the same block.  `skip`: nothing is written when it is set.
+template <int N, bool TRI>
+__global__ __launch_bounds__(256) void rotate_kernel(const double* src, int64_t lds, double* dst,
+                                                     int64_t ldd, int64_t D, int n,
+                                                     const double* __restrict__ M,
+                                                     const int* __restrict__ skip) {
+  __shared__ double sM[N * N];
+  if (skip && *skip) return;  // (uniform)
+  for (int i = threadIdx.x; i < n * n; i += blockDim.x) sM[(i / n) * N + i % n] = M[i];
   __syncthreads();
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= D) return;
-  double row[kMaxN];
-#pragma unroll 8
-  for (int i = 0; i < n; ++i) row[i] = W[r + (int64_t)i * ldw];
-  for (int j = 0; j < n; ++j) {
-    double t = 0.0;
-    for (int i = 0; i < n; ++i) t += row[i] * sM[i + j * n];
-    W[r + (int64_t)j * ldw] = t;
+  double row[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) row[i] = i < n ? src[r + (int64_t)i * lds] : 0.0;
+  if constexpr (TRI) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (j >= n) break;
+      double t = 0.0;
+#pragma unroll
+      for (int i = 0; i <= j; ++i) t += row[i] * sM[i + j * N];
+      dst[r + (int64_t)j * ldd] = t;
+    }
+  } else {
+    for (int j = 0; j < n; ++j) {
+      double t = 0.0;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (i < n) t += row[i] * sM[i + j * N];
+      dst[r + (int64_t)j * ldd] = t;
+    }
   }
+}
+
+// One pass of Cholesky-QR in one block: G = W^T W from the Gram partials (nrb > 0) or
+// already summed in `part`, its factor R (G = R^T R) to Rout, R^-1 to Ri (both n x n,
+// column-major, upper).  With Rin (the second pass) Rout gets R * Rin.  A pivot that
+// is not positive and finite sets *fail (and *fail_host), and so does a set *prev;
+// every product is rounded (no fused multiply-add), so that the pivot of a repeated
+// column cancels to zero.
+__global__ __launch_bounds__(1024) void chol_kernel(const double* __restrict__ part, int nrb, int n,
+                                                    const double* __restrict__ Rin,
+                                                    double* Rout, double* __restrict__ Ri,
+                                                    const int* prev, int* fail,
+                                                    int* fail_host) {
+#pragma clang fp contract(off)
+  extern __shared__ double chol_lds[];
+  double* G = chol_lds;             // G, then R (row j from column j on)
+  double* I = chol_lds + n * n;     // partial sums, then the inverse
+  const int t = threadIdx.x, nn = n * n;
+  auto end = [&](int v) {
+    if (t != 0) return;
+    *fail = v;
+    if (fail_host) *fail_host = v;
+  };
+  if (prev && *prev) return end(1);  // (uniform)
+  if (nrb > 0) {  // n <= 16: the threads of an entry add their partials, then one adds these
+    const int g = 1024 / nn, e = t / g, k = t % g;
+    double v = 0.0;
+    if (e < nn)
+      for (int rb = k; rb < nrb; rb += 8 * g) {  // (eight loads in flight)
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          x[u] = rb + u * g < nrb ? part[(int64_t)(rb + u * g) * nn + e] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v += x[u];
+      }
+    I[t] = v;
+    __syncthreads();
+    if (t < nn) {
+      double sum = 0.0;
+      for (int i = 0; i < g; ++i) sum += I[t * g + i];
+      G[t] = sum;
+    }
+  } else {
+    for (int i = t; i < nn; i += 1024) G[i] = part[i];
+  }
+  __syncthreads();
+  const int nt = n <= 16 ? 64 : 1024;  // (one wave: its barriers cost nothing)
+  if (t >= nt) return;
+  for (int j = 0; j < n; ++j) {
+    const double d = G[j * n + j];
+    if (!(d > 0.0) || d > 1.7976931348623157e308) return end(1);  // (uniform)
+    const double r = sqrt(d);
+    __syncthreads();
+    if (t == 0) G[j * n + j] = r;
+    else if (j + t < n) G[j * n + j + t] /= r;
+    __syncthreads();
+    const int m = n - 1 - j;
+    for (int i = t; i < m * m; i += nt) {
+      const int a = j + 1 + i / m, b = j + 1 + i % m;
+      if (b >= a) G[a * n + b] -= G[j * n + a] * G[j * n + b];
+    }
+    __syncthreads();
+  }
+  if (t < n) {  // column t of the inverse
+    I[t * n + t] = 1.0 / G[t * n + t];
+    for (int i = t - 1; i >= 0; --i) {
+      double v = 0.0;
+      for (int k = i + 1; k <= t; ++k) v += G[i * n + k] * I[t * n + k];
+      I[t * n + i] = -v / G[i * n + i];
+    }
+    for (int i = t + 1; i < n; ++i) I[t * n + i] = 0.0;
+  }
+  __syncthreads();
+  for (int e = t; e < nn; e += nt) {
+    const int i = e % n, j = e / n;
+    Ri[e] = I[e];
+    double v = 0.0;
+    if (i <= j) {
+      if (Rin)
+        for (int k = i; k <= j; ++k) v += G[i * n + k] * Rin[k + j * n];
+      else v = G[i * n + j];
+    }
+    Rout[e] = v;
+  }
+  end(0);
 }
 
 // Column partials of <A_j, B_j> (mode 0) or ||A_j - e_j B_j||^2 (mode 1).
@@ -250,30 +384,27 @@ __global__ __launch_bounds__(256) void coldot_kernel(const double* __restrict__ 
   if (threadIdx.x == 0) part[(int64_t)c * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-__global__ void copy_block_kernel(const double* __restrict__ src, int64_t lds, double* __restrict__ dst,
-                                  int64_t ldd, int64_t D) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int c = blockIdx.y;
-  if (r < D) dst[r + (int64_t)c * ldd] = src[r + (int64_t)c * lds];
-}
-
 // ---------------------------------------------------------------- drivers
 // G(i, j) = <A_i, B_j> stored at G[i*gsi + j*gsj] (column-major: gsi = 1,
 // gsj = ldg >= m; row-major: gsi = ldg >= n, gsj = 1).
-void gram(pf_handle* h, const double* A, int64_t lda, int m, const double* B, int64_t ldb, int n,
-          int64_t D, double* G, int64_t gsi, int64_t gsj, hipStream_t st) {
-  PF_REQUIRE(m >= 1 && n >= 1 && n <= kMaxN, "gram: 1 <= n <= 64, m >= 1");
-  PF_REQUIRE(D >= 1 && lda >= D && ldb >= D, "gram: bad leading dimensions");
-  PF_REQUIRE((gsi == 1 && gsj >= m) || (gsj == 1 && gsi >= n), "gram: bad output layout");
-  const int nrb = (int)std::min<int64_t>(kGramRowBlocks, (D + 15) / 16);
+static int gram_partials(pf_handle* h, const double* A, int64_t lda, int m, const double* B,
+                         int64_t ldb, int n, int64_t D, hipStream_t st) {
+  const int nrb = (int)std::min<int64_t>(m <= 16 ? kGramRowBlocks1 : kGramRowBlocks, (D + 15) / 16);
   double* part = reinterpret_cast<double*>(h->partials.get((size_t)nrb * m * n * sizeof(double)));
   // two A tiles per wave once A is wider than one block's 64 columns
   const int AT = m > 64 ? 2 : 1;
   dim3 grid(nrb, (m + 64 * AT - 1) / (64 * AT)), block(256);
   const int NT = (n + 15) / 16;
-#define PF_GRAM(NTV, ATV) \
-  hipLaunchKernelGGL((gram_kernel<NTV, ATV>), grid, block, 0, st, A, lda, m, B, ldb, n, D, part)
-  if (AT == 2) {
+#define PF_GRAM(...) \
+  hipLaunchKernelGGL((gram_kernel<__VA_ARGS__>), grid, block, 0, st, A, lda, m, B, ldb, n, D, part)
+  if (m <= 16) {
+    switch (NT) {
+      case 1: PF_GRAM(1, 1, true); break;
+      case 2: PF_GRAM(2, 1, true); break;
+      case 3: PF_GRAM(3, 1, true); break;
+      default: PF_GRAM(4, 1, true); break;
+    }
+  } else if (AT == 2) {
     switch (NT) {
       case 1: PF_GRAM(1, 2); break;
       case 2: PF_GRAM(2, 2); break;
@@ -290,8 +421,17 @@ void gram(pf_handle* h, const double* A, int64_t lda, int m, const double* B, in
   }
 #undef PF_GRAM
   PF_HIP(hipGetLastError());
+  return nrb;
+}
+void gram(pf_handle* h, const double* A, int64_t lda, int m, const double* B, int64_t ldb, int n,
+          int64_t D, double* G, int64_t gsi, int64_t gsj, hipStream_t st) {
+  PF_REQUIRE(m >= 1 && n >= 1 && n <= kMaxN, "gram: 1 <= n <= 64, m >= 1");
+  PF_REQUIRE(D >= 1 && lda >= D && ldb >= D, "gram: bad leading dimensions");
+  PF_REQUIRE((gsi == 1 && gsj >= m) || (gsj == 1 && gsi >= n), "gram: bad output layout");
+  const int nrb = gram_partials(h, A, lda, m, B, ldb, n, D, st);
+  const double* part = reinterpret_cast<const double*>(h->partials.p);
   const int64_t mn = (int64_t)m * n;
-  hipLaunchKernelGGL(gram_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, part,
+  hipLaunchKernelGGL(gram_reduce_kernel, dim3((unsigned)((mn + 31) / 32)), dim3(256), 0, st, part,
                      nrb, m, n, G, gsi, gsj);
   PF_HIP(hipGetLastError());
 }
@@ -337,36 +477,20 @@ static void coldots_host(pf_handle* h, const double* A, int64_t lda, const doubl
   }
 }
 
-// Cholesky G = R^T R of a small SPD matrix (column-major, n x n); returns false
-// when a pivot is not positive.
-static bool cholesky_upper(const std::vector<double>& G, int n, std::vector<double>& R) {
-  R.assign((size_t)n * n, 0.0);
-  for (int j = 0; j < n; ++j) {
-    double d = G[j + (size_t)j * n];
-    for (int k = 0; k < j; ++k) d -= R[k + (size_t)j * n] * R[k + (size_t)j * n];
-    if (!(d > 0.0) || !std::isfinite(d)) return false;
-    const double rjj = std::sqrt(d);
-    R[j + (size_t)j * n] = rjj;
-    for (int i = j + 1; i < n; ++i) {
-      double t = G[j + (size_t)i * n];
-      for (int k = 0; k < j; ++k) t -= R[k + (size_t)j * n] * R[k + (size_t)i * n];
-      R[j + (size_t)i * n] = t / rjj;
-    }
-  }
-  return true;
-}
-
-// inverse of an upper-triangular n x n matrix (column-major)
-static void inv_upper(const std::vector<double>& R, int n, std::vector<double>& Ri) {
-  Ri.assign((size_t)n * n, 0.0);
-  for (int j = 0; j < n; ++j) {
-    Ri[j + (size_t)j * n] = 1.0 / R[j + (size_t)j * n];
-    for (int i = j - 1; i >= 0; --i) {
-      double t = 0.0;
-      for (int k = i + 1; k <= j; ++k) t += R[i + (size_t)k * n] * Ri[k + (size_t)j * n];
-      Ri[i + (size_t)j * n] = -t / R[i + (size_t)i * n];
-    }
-  }
+template <bool TRI>
+static void rotate_launch(const double* src, int64_t lds, double* dst, int64_t ldd, int64_t D,
+                          int n, const double* M, const int* skip, hipStream_t st) {
+  const dim3 grid((unsigned)((D + 255) / 256)), block(256);
+#define PF_ROTATE(N) \
+  hipLaunchKernelGGL((rotate_kernel<N, TRI>), grid, block, 0, st, src, lds, dst, ldd, D, n, M, skip)
+  if (n == 1) PF_ROTATE(1);
+  else if (n <= 4) PF_ROTATE(4);
+  else if (n <= 8) PF_ROTATE(8);
+  else if (n <= 16) PF_ROTATE(16);
+  else if (n <= 32) PF_ROTATE(32);
+  else PF_ROTATE(64);
+#undef PF_ROTATE
+  PF_HIP(hipGetLastError());
 }
 
 static void rotate(pf_handle* h, double* W, int64_t ldw, int64_t D, int n, const double* M_host,
@@ -374,9 +498,7 @@ static void rotate(pf_handle* h, double* W, int64_t ldw, int64_t D, int n, const
   PF_REQUIRE(n >= 1 && n <= kMaxN, "rotate: 1 <= n <= 64");
   double* dM = reinterpret_cast<double*>(h->small.get((size_t)n * n * sizeof(double)));
   PF_HIP(hipMemcpyAsync(dM, M_host, (size_t)n * n * sizeof(double), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(rotate_kernel, dim3((unsigned)((D + 255) / 256)), dim3(256), 0, st, W, ldw, D,
-                     n, dM);
-  PF_HIP(hipGetLastError());
+  rotate_launch<false>(W, ldw, W, ldw, D, n, dM, nullptr, st);
   // the host matrix may be freed by the caller after return
   PF_HIP(hipStreamSynchronize(st));
 }
@@ -428,37 +550,38 @@ extern "C" int pf_block_qr(pf_handle* h, double* W, int64_t ldw, int64_t D, int3
     PF_REQUIRE(h && W && R_host, "qr: null argument");
     PF_REQUIRE(s >= 1 && s <= kMaxN && D >= s && ldw >= D, "qr: bad shape");
     hipStream_t st = S(stream);
-    // keep a copy to restore W when Cholesky breaks down
-    double* save = reinterpret_cast<double*>(
-        h->vecs.get((size_t)D * s * sizeof(double) + (size_t)s * s * sizeof(double)));
-    double* dG = save + (size_t)D * s;
-    hipLaunchKernelGGL(copy_block_kernel, dim3((unsigned)((D + 255) / 256), s), dim3(256), 0, st, W,
-                       ldw, save, D, D);
-    PF_HIP(hipGetLastError());
-    std::vector<double> G((size_t)s * s), R1, R2, Ri, R((size_t)s * s, 0.0);
+    // Two passes on the device, the first into a copy, so that W is unchanged when a
+    // factorization breaks down; R and the flags go straight to pinned host memory,
+    // and the one wait is at the end.
+    if (!h->pinned)
+      PF_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->pinned),
+                           ((size_t)kMaxN * kMaxN + 2) * sizeof(double)));
+    const size_t ss = (size_t)s * s;
+    double* Q = reinterpret_cast<double*>(h->vecs.get(((size_t)D * s + 3 * ss + 2) * sizeof(double)));
+    double* dG = Q + (size_t)D * s;
+    double *R1 = dG + ss, *Ri = R1 + ss;
+    int* flag = reinterpret_cast<int*>(Ri + ss);
+    int* flag_host = reinterpret_cast<int*>(h->pinned + ss);
     for (int pass = 0; pass < 2; ++pass) {
-      gram(h, W, ldw, s, W, ldw, s, D, dG, 1, s, st);
-      PF_HIP(hipMemcpyAsync(G.data(), dG, G.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-      PF_HIP(hipStreamSynchronize(st));
-      std::vector<double>& Rp = pass == 0 ? R1 : R2;
-      if (!cholesky_upper(G, s, Rp)) {
-        hipLaunchKernelGGL(copy_block_kernel, dim3((unsigned)((D + 255) / 256), s), dim3(256), 0,
-                           st, save, D, W, ldw, D);
-        PF_HIP(hipGetLastError());
-        PF_HIP(hipStreamSynchronize(st));
-        throw Error{PF_ERR_NUMERIC, "qr: Gram matrix not positive definite (rank-deficient block)"};
-      }
-      inv_upper(Rp, s, Ri);
-      rotate(h, W, ldw, D, s, Ri.data(), st);
+      const double* A = pass ? Q : W;
+      const int64_t lda = pass ? D : ldw;
+      const bool fused = s <= 16;
+      int nrb = 0;
+      if (fused) nrb = gram_partials(h, A, lda, s, A, lda, s, D, st);
+      else gram(h, A, lda, s, A, lda, s, D, dG, 1, s, st);
+      const size_t lds = std::max(2 * ss, ss + 1024) * sizeof(double);
+      hipLaunchKernelGGL(chol_kernel, dim3(1), dim3(1024), lds, st,
+                         fused ? reinterpret_cast<const double*>(h->partials.p) : dG, nrb, s,
+                         pass ? R1 : nullptr, pass ? h->pinned : R1, Ri, pass ? flag : nullptr,
+                         flag + pass, pass ? flag_host : nullptr);
+      PF_HIP(hipGetLastError());
+      if (pass == 0) rotate_launch<true>(W, ldw, Q, D, D, s, Ri, flag, st);
+      else rotate_launch<true>(Q, D, W, ldw, D, s, Ri, flag + 1, st);
     }
-    // R = R2 * R1 (both upper triangular)
-    for (int j = 0; j < s; ++j)
-      for (int i = 0; i <= j; ++i) {
-        double t = 0.0;
-        for (int k = i; k <= j; ++k) t += R2[i + (size_t)k * s] * R1[k + (size_t)j * s];
-        R[i + (size_t)j * s] = t;
-      }
-    std::memcpy(R_host, R.data(), R.size() * sizeof(double));
+    PF_HIP(hipStreamSynchronize(st));
+    if (*flag_host)
+      throw Error{PF_ERR_NUMERIC, "qr: Gram matrix not positive definite (rank-deficient block)"};
+    std::memcpy(R_host, h->pinned, ss * sizeof(double));
   });
 }
 

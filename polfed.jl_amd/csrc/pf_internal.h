@@ -171,6 +171,7 @@ struct pf_handle {
   pf::DevBuf partials;  // gram partial sums
   pf::DevBuf small;     // small matrices staged to the device
   pf::DevBuf vecs;      // residual / rotation scratch
+  double* pinned = nullptr;  // results of a QR, written by its kernels
 };
 
 struct pf_op {

@@ -1,0 +1,39 @@
+"""Cholesky-QR on the device (csrc/dense.hip) against numpy's QR: block widths at the
+edges of its register and reduction variants, padded leading dimensions, and blocks
+whose first or second factorization breaks down."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("s", [1, 2, 4, 5, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("D", [70, 5003])
+def test_block_qr_matches_numpy(dev, s, D):
+    from polfed_amd import NumericBreakdown
+    from polfed_amd import blockops as bo
+    rng = np.random.default_rng(s + D)
+    W = rng.standard_normal((D, s)) * np.logspace(0, -3, s)
+    pad = torch.full((s, D + 5), np.nan, dtype=torch.float64, device=dev.torch_device)
+    pad[:, :D] = dev.to_device(W)
+    Q = pad[:, :D]
+    R = bo.block_qr(dev, Q)
+    Qn, Rn = np.linalg.qr(W)
+    sign = np.sign(np.diag(Rn))
+    q = dev.to_host(Q)
+    # two passes: orthogonal to a few roundings of D-term sums
+    assert np.max(np.abs(q.T @ q - np.eye(s))) < 1e-13
+    assert np.max(np.abs(q - Qn * sign)) < 1e-10
+    assert np.max(np.abs(R - Rn * sign[:, None])) < 1e-11 * np.max(np.abs(Rn))
+    assert np.array_equal(R, np.triu(R))
+    assert torch.isnan(pad[:, D:]).all()
+    bad = [np.zeros((D, s)), np.full((D, s), np.inf)]
+    if s > 1:
+        bad.append(np.repeat(W[:, :1], s, axis=1) * np.where(np.arange(s) == s - 1, 0.0, 1.0))
+    for B in bad:
+        Bd = dev.to_device(B)
+        keep = Bd.clone()
+        with pytest.raises(NumericBreakdown):
+            bo.block_qr(dev, Bd)
+        assert torch.equal(Bd, keep)
