@@ -296,6 +296,15 @@ int pf_reorth(pf_handle* h, const double* V, int64_t ldv, int32_t k, double* W, 
 int pf_block_qr(pf_handle* h, double* W, int64_t ldw, int64_t D, int32_t s, double* R_host,
                 pf_stream stream);
 
+/* Orthogonalization of a three-term block step, s <= 16: a = the upper triangle of
+ * V^T W mirrored (to a_host, s x s column-major), then W -= V a and, unless Vp is
+ * null, W -= Vp b^T with b = b_host (s x s column-major).  Returns when a_host is
+ * there; the updates of W follow on the stream.  calcoverlap!
+ * (BlockLanczosFactorization.jl:102-111) and the orthogonalization in one call. */
+int pf_lanczos_ortho(pf_handle* h, const double* V, int64_t ldv, const double* Vp, int64_t ldvp,
+                     const double* b_host, double* W, int64_t ldw, int64_t D, int32_t s,
+                     double* a_host, pf_stream stream);
+
 /* W <- W * M for a small n x n matrix M (host, column-major), row by row in
  * place (used to apply R^{-1} or a basis rotation). */
 int pf_rotate(pf_handle* h, double* W, int64_t ldw, int64_t D, int32_t n, const double* M_host,

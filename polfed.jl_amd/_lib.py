@@ -110,6 +110,8 @@ SIGNATURES = {
     "pf_gemm_update": (_c.c_int, [_vp, _vp, _i64, _i32, _vp, _i32, _vp, _i64, _i32, _i64, _dbl,
                                   _dbl, _vp]),
     "pf_reorth": (_c.c_int, [_vp, _vp, _i64, _i32, _vp, _i64, _i32, _i64, _i32, _vp]),
+    "pf_lanczos_ortho": (_c.c_int, [_vp, _vp, _i64, _vp, _i64, _pdbl, _vp, _i64, _i64, _i32, _pdbl,
+                                    _vp]),
     "pf_block_qr": (_c.c_int, [_vp, _vp, _i64, _i64, _i32, _pdbl, _vp]),
     "pf_rotate": (_c.c_int, [_vp, _vp, _i64, _i64, _i32, _pdbl, _vp]),
     "pf_residuals": (_c.c_int, [_vp, _vp, _vp, _i64, _i32, _pdbl, _pdbl, _vp]),

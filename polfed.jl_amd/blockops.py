@@ -66,6 +66,35 @@ def block_qr(dev: Device, W: torch.Tensor) -> np.ndarray:
     return R
 
 
+def lanczos_ortho(dev: Device, V: torch.Tensor, Vprev: torch.Tensor | None,
+                  b: np.ndarray | None, W: torch.Tensor) -> np.ndarray:
+    """W -= V a + Vprev b^T with a = the upper triangle of V^T W mirrored, which is
+    returned (s x s); Vprev and b may be None.  One call for blocks of up to 16
+    columns; it returns while the updates of W are still running."""
+    pv, ldv, D, s = colmajor(V)
+    pw, ldw, D2, s2 = colmajor(W)
+    if D != D2 or s != s2 or (Vprev is not None and Vprev.shape != V.shape):
+        raise ValueError("lanczos_ortho: shape mismatch")
+    if s > 16:
+        a = gram(dev, V, W).cpu().numpy().T
+        a = np.triu(a) + np.triu(a, 1).T
+        col = lambda m: torch.as_tensor(np.ascontiguousarray(m.T), device=W.device)
+        update(dev, V, col(a), W, alpha=-1.0, beta=1.0)
+        if Vprev is not None:
+            update(dev, Vprev, col(b.T), W, alpha=-1.0, beta=1.0)
+        return a
+    a = np.empty((s, s), order="F")
+    pp = bp = None
+    ldp = 0
+    if Vprev is not None:
+        pp, ldp = colmajor(Vprev)[:2]
+        bf = np.asfortranarray(b, dtype=np.float64)
+        bp = bf.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    check(dev.lib.pf_lanczos_ortho(dev.h, pv, ldv, pp, ldp, bp, pw, ldw, D, s,
+                                   a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), dev.stream))
+    return a
+
+
 def rotate(dev: Device, W: torch.Tensor, M: np.ndarray) -> None:
     """W <- W M in place for a small n x n host matrix M."""
     pw, ldw, D, n = colmajor(W)

@@ -46,6 +46,7 @@ extern "C" int pf_destroy(pf_handle* h) {
   h->small.release();
   h->vecs.release();
   if (h->pinned) (void)hipHostFree(h->pinned);
+  if (h->mark) (void)hipEventDestroy(h->mark);
   delete h;
   return PF_OK;
 }

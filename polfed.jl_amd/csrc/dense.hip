@@ -273,6 +273,32 @@ __global__ __launch_bounds__(256) void rotate_kernel(const double* src, int64_t 
   }
 }
 
+// G = the sums of nrb partials of nn <= 256 entries, in one block of 1024 threads (I:
+// 1024 doubles): the threads of an entry add their partials, eight loads in flight,
+// then one adds these.
+__device__ __forceinline__ void sum_partials(const double* __restrict__ part, int nrb, int nn,
+                                             double* I, double* G) {
+  const int t = threadIdx.x, g = 1024 / nn, e = t / g, k = t % g;
+  double v = 0.0;
+  if (e < nn)
+    for (int rb = k; rb < nrb; rb += 8 * g) {
+      double x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        x[u] = rb + u * g < nrb ? part[(int64_t)(rb + u * g) * nn + e] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v += x[u];
+    }
+  I[t] = v;
+  __syncthreads();
+  if (t < nn) {
+    double sum = 0.0;
+    for (int i = 0; i < g; ++i) sum += I[t * g + i];
+    G[t] = sum;
+  }
+  __syncthreads();
+}
+
 // One pass of Cholesky-QR in one block: G = W^T W from the Gram partials (nrb > 0) or
 // already summed in `part`, its factor R (G = R^T R) to Rout, R^-1 to Ri (both n x n,
 // column-major, upper).  With Rin (the second pass) Rout gets R * Rin.  A pivot that
@@ -295,25 +321,8 @@ __global__ __launch_bounds__(1024) void chol_kernel(const double* __restrict__ p
     if (fail_host) *fail_host = v;
   };
   if (prev && *prev) return end(1);  // (uniform)
-  if (nrb > 0) {  // n <= 16: the threads of an entry add their partials, then one adds these
-    const int g = 1024 / nn, e = t / g, k = t % g;
-    double v = 0.0;
-    if (e < nn)
-      for (int rb = k; rb < nrb; rb += 8 * g) {  // (eight loads in flight)
-        double x[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          x[u] = rb + u * g < nrb ? part[(int64_t)(rb + u * g) * nn + e] : 0.0;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v += x[u];
-      }
-    I[t] = v;
-    __syncthreads();
-    if (t < nn) {
-      double sum = 0.0;
-      for (int i = 0; i < g; ++i) sum += I[t * g + i];
-      G[t] = sum;
-    }
+  if (nrb > 0) {  // n <= 16
+    sum_partials(part, nrb, nn, I, G);
   } else {
     for (int i = t; i < nn; i += 1024) G[i] = part[i];
   }
@@ -357,6 +366,26 @@ __global__ __launch_bounds__(1024) void chol_kernel(const double* __restrict__ p
     Rout[e] = v;
   }
   end(0);
+}
+
+// The projections of a three-term step in one block (n <= 16): G = V^T W from its
+// partials, a = its upper triangle mirrored, to `a` and to pinned host memory, and
+// the transpose of b (by value) to `bt`; all column-major.
+struct OrthoB {
+  double v[16 * 16];
+};
+__global__ __launch_bounds__(1024) void ortho_kernel(const double* __restrict__ part, int nrb,
+                                                     int n, const OrthoB b, double* a, double* bt,
+                                                     double* a_host) {
+  __shared__ double I[1024], G[256];
+  const int t = threadIdx.x, nn = n * n;
+  sum_partials(part, nrb, nn, I, G);
+  if (t >= nn) return;
+  const int i = t % n, j = t / n;
+  const double v = G[(i < j ? i : j) * n + (i < j ? j : i)];
+  a[t] = v;
+  a_host[t] = v;
+  bt[t] = b.v[t];
 }
 
 // Column partials of <A_j, B_j> (mode 0) or ||A_j - e_j B_j||^2 (mode 1).
@@ -493,6 +522,13 @@ static void rotate_launch(const double* src, int64_t lds, double* dst, int64_t l
   PF_HIP(hipGetLastError());
 }
 
+// Pinned results of the small factorizations: kMaxN^2 doubles and a flag.
+static void qr_pinned(pf_handle* h) {
+  if (!h->pinned)
+    PF_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->pinned),
+                         ((size_t)kMaxN * kMaxN + 2) * sizeof(double)));
+}
+
 static void rotate(pf_handle* h, double* W, int64_t ldw, int64_t D, int n, const double* M_host,
                    hipStream_t st) {
   PF_REQUIRE(n >= 1 && n <= kMaxN, "rotate: 1 <= n <= 64");
@@ -553,9 +589,7 @@ extern "C" int pf_block_qr(pf_handle* h, double* W, int64_t ldw, int64_t D, int3
     // Two passes on the device, the first into a copy, so that W is unchanged when a
     // factorization breaks down; R and the flags go straight to pinned host memory,
     // and the one wait is at the end.
-    if (!h->pinned)
-      PF_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->pinned),
-                           ((size_t)kMaxN * kMaxN + 2) * sizeof(double)));
+    qr_pinned(h);
     const size_t ss = (size_t)s * s;
     double* Q = reinterpret_cast<double*>(h->vecs.get(((size_t)D * s + 3 * ss + 2) * sizeof(double)));
     double* dG = Q + (size_t)D * s;
@@ -582,6 +616,35 @@ extern "C" int pf_block_qr(pf_handle* h, double* W, int64_t ldw, int64_t D, int3
     if (*flag_host)
       throw Error{PF_ERR_NUMERIC, "qr: Gram matrix not positive definite (rank-deficient block)"};
     std::memcpy(R_host, h->pinned, ss * sizeof(double));
+  });
+}
+
+extern "C" int pf_lanczos_ortho(pf_handle* h, const double* V, int64_t ldv, const double* Vp,
+                                int64_t ldvp, const double* b_host, double* W, int64_t ldw,
+                                int64_t D, int32_t s, double* a_host, pf_stream stream) {
+  return guarded([&] {
+    PF_REQUIRE(h && V && W && a_host && (!Vp || b_host), "ortho: null argument");
+    PF_REQUIRE(s >= 1 && s <= 16 && D >= 1 && ldv >= D && ldw >= D && (!Vp || ldvp >= D),
+               "ortho: bad shape");
+    PF_REQUIRE(V != W && Vp != W, "ortho: W must not alias V");
+    hipStream_t st = S(stream);
+    double* a = reinterpret_cast<double*>(h->small.get(2 * 256 * sizeof(double)));
+    double* bt = a + 256;
+    qr_pinned(h);
+    if (!h->mark) PF_HIP(hipEventCreateWithFlags(&h->mark, hipEventDisableTiming));
+    OrthoB b{};
+    if (Vp)
+      for (int i = 0; i < s; ++i)
+        for (int j = 0; j < s; ++j) b.v[j + i * s] = b_host[i + j * s];
+    const int nrb = gram_partials(h, V, ldv, s, W, ldw, s, D, st);
+    hipLaunchKernelGGL(ortho_kernel, dim3(1), dim3(1024), 0, st,
+                       reinterpret_cast<const double*>(h->partials.p), nrb, s, b, a, bt, h->pinned);
+    PF_HIP(hipGetLastError());
+    PF_HIP(hipEventRecord(h->mark, st));
+    update(V, ldv, s, a, 1, s, W, ldw, s, D, -1.0, 1.0, st);
+    if (Vp) update(Vp, ldvp, s, bt, 1, s, W, ldw, s, D, -1.0, 1.0, st);
+    PF_HIP(hipEventSynchronize(h->mark));  // (the updates are still running)
+    std::memcpy(a_host, h->pinned, (size_t)s * s * sizeof(double));
   });
 }
 

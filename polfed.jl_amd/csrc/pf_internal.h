@@ -171,7 +171,8 @@ struct pf_handle {
   pf::DevBuf partials;  // gram partial sums
   pf::DevBuf small;     // small matrices staged to the device
   pf::DevBuf vecs;      // residual / rotation scratch
-  double* pinned = nullptr;  // results of a QR, written by its kernels
+  double* pinned = nullptr;  // small results, written by their kernels
+  hipEvent_t mark = nullptr; // when such a result is there
 };
 
 struct pf_op {

@@ -102,26 +102,29 @@ def _host_qr(block: torch.Tensor) -> np.ndarray:
     return R
 
 
+class _Stage:
+    def __init__(self, timer, key):
+        self.timer, self.key = timer, key
+
+    def __enter__(self):
+        if self.timer.sync:
+            torch.cuda.synchronize()
+        self.t0 = time.perf_counter()
+
+    def __exit__(self, *a):
+        if self.timer.sync:
+            torch.cuda.synchronize()
+        t = self.timer.t
+        t[self.key] = t.get(self.key, 0.0) + time.perf_counter() - self.t0
+
+
 class _Timer:
     def __init__(self, sync: bool):
         self.sync = sync
         self.t = {}
 
     def __call__(self, key):
-        timer = self
-
-        class _Ctx:
-            def __enter__(self):
-                if timer.sync:
-                    torch.cuda.synchronize()
-                self.t0 = time.perf_counter()
-
-            def __exit__(self, *a):
-                if timer.sync:
-                    torch.cuda.synchronize()
-                timer.t[key] = timer.t.get(key, 0.0) + time.perf_counter() - self.t0
-
-        return _Ctx()
+        return _Stage(self, key)
 
 
 def lanczos(dev: Device, f, x0: torch.Tensor, howmany: int, *, maxdim: int | None = None,
@@ -227,12 +230,6 @@ def lanczos_coroutine(dev: Device, x0: torch.Tensor, howmany: int, *,
     mat = np.zeros((maxdim, maxdim))
     r = torch.empty((s, D), dtype=torch.float64, device=X0.device)
 
-    def sym_upper(a):
-        return np.triu(a) + np.triu(a, 1).T
-
-    def overlap(V, W):
-        return bo.gram(dev, V, W).cpu().numpy().T
-
     # ---- lanczositer (Factorization.jl:50-67)
     V0 = basis.block(0)
     V0.copy_(X0)
@@ -240,10 +237,9 @@ def lanczos_coroutine(dev: Device, x0: torch.Tensor, howmany: int, *,
     k = s
     with tm("mapping"):
         yield V0, r, False
-    a = sym_upper(overlap(V0, r))
+    a = bo.lanczos_ortho(dev, V0, None, None, r)
     mat[0:s, 0:s] = a
     tmax = float(np.max(np.abs(a)))  # max|mat| so far
-    bo.update(dev, V0, _to_dev_matrix(a, r), r, alpha=-1.0, beta=1.0)
     numiter = 1
     nextcheck = max(howmany // s + 1, 2)
     converged = eigenconverged = 0
@@ -360,12 +356,9 @@ def lanczos_coroutine(dev: Device, x0: torch.Tensor, howmany: int, *,
                 fast_iters += 1
         # [3] calculate_overlap!  [4] orthogonalization!
         with tm("orthogonalization"):
-            a = sym_upper(overlap(V_last, r))
+            a = bo.lanczos_ortho(dev, V_last, V_prev, mat[k - s:k, k - 2 * s:k - s], r)
             mat[k - s:k, k - s:k] = a
             tmax = max(tmax, float(np.max(np.abs(a))))
-            b = mat[k - s:k, k - 2 * s:k - s]
-            bo.update(dev, V_last, _to_dev_matrix(a, r), r, alpha=-1.0, beta=1.0)
-            bo.update(dev, V_prev, _to_dev_matrix(b.T, r), r, alpha=-1.0, beta=1.0)
         # [5] reorthogonalization! against all but the last two blocks
         with tm("reorthogonalization"):
             nb = k - 2 * s

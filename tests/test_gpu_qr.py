@@ -1,6 +1,7 @@
 """Cholesky-QR on the device (csrc/dense.hip) against numpy's QR: block widths at the
 edges of its register and reduction variants, padded leading dimensions, and blocks
-whose first or second factorization breaks down."""
+whose first or second factorization breaks down; the three-term projection of a
+block step against numpy."""
 import numpy as np
 import pytest
 import torch
@@ -37,3 +38,20 @@ def test_block_qr_matches_numpy(dev, s, D):
         with pytest.raises(NumericBreakdown):
             bo.block_qr(dev, Bd)
         assert torch.equal(Bd, keep)
+
+
+@pytest.mark.parametrize("s", [1, 3, 8, 16, 17])
+@pytest.mark.parametrize("D", [40, 5003])
+def test_lanczos_ortho_matches_numpy(dev, s, D):
+    from polfed_amd import blockops as bo
+    rng = np.random.default_rng(s + D)
+    V, Vp, W, B = (rng.standard_normal((D, s)) / np.sqrt(D) for _ in range(4))
+    b = np.triu(B[:s])
+    a = V.T @ W
+    a = np.triu(a) + np.triu(a, 1).T
+    for prev in (False, True):
+        Wd = dev.to_device(W)
+        got = bo.lanczos_ortho(dev, dev.to_device(V), dev.to_device(Vp) if prev else None,
+                               b if prev else None, Wd)
+        assert np.max(np.abs(got - a)) < 1e-14
+        assert np.max(np.abs(dev.to_host(Wd) - (W - V @ a - (Vp @ b.T if prev else 0.0)))) < 1e-14
