@@ -26,21 +26,22 @@ __device__ __forceinline__ d4 mfma16x16x4(double a, double b, d4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// row partitions of the Gram reduction: two blocks per CU and 128 columns of a wide A
-// (614 MB: 170 us with 128, 161 so), half of it for one tile of columns, whose
-// partials one block adds up
+// Row partitions of the Gram reduction, each a contiguous range of rows (616 MB, 416
+// columns: 162 us with every 256th slab, 136 so; 145 with 128 ranges of twice the
+// columns per wave, 153 with 512), half of it for one tile of columns, whose
+// partials one block adds up.
 constexpr int kGramRowBlocks = 256, kGramRowBlocks1 = 128;
 constexpr int kMaxN = 64;            // widest B block of the Gram/update kernels
 
-// WS: A has at most 16 columns; the four waves take every fourth slab each and add
+// WS: A has at most 16 columns; the four waves take a quarter of the slabs each and add
 // their tiles in LDS (184756 x 8: 28.4 us with three waves idle, 10.1 us so).
 //
 // Gram partials: part[(rb * m + i) * n + j] = sum over rb's slabs of A[:, i] B[:, j].
 // Grid: (kGramRowBlocks, ceil(m/(64*AT))); block: 4 waves, wave w owns the AT
 // tiles of 16 A columns from i0 = 64*AT*blockIdx.y + 16*AT*w and all n columns
-// of B (NT <= 4 tiles), so each B load serves AT A tiles.  Slab sl (16 rows)
-// belongs to row block sl mod gridDim.x; a block takes its full slabs two at
-// a time with every load issued before the first MFMA.  Lanes past m or n
+// of B (NT <= 4 tiles), so each B load serves AT A tiles.  Row block rb
+// takes a contiguous range of slabs (16 rows), two at a time with every load issued
+// before the first MFMA.  Lanes past m or n
 // read a clamped column (their results are not stored); only the rows past D
 // of the last, partial slab are zeroed.
 template <int NT, int AT, bool WS = false>
@@ -89,20 +90,21 @@ __global__ __launch_bounds__(256) void gram_kernel(const double* __restrict__ A,
   };
   const int64_t gx = WS ? 4 * gridDim.x : gridDim.x, nfull = D / 16;
   const int64_t first = WS ? 4 * blockIdx.x + w : blockIdx.x;
-  int64_t sl = first;
-  for (; sl + gx < nfull; sl += 2 * gx) {
+  const int64_t end = (first + 1) * nfull / gx;
+  int64_t sl = first * nfull / gx;
+  for (; sl + 1 < end; sl += 2) {
     double av0[AT][4], bv0[NT][4], av1[AT][4], bv1[NT][4];
     load(sl * 16 + 4 * kq, false, av0, bv0);
-    load((sl + gx) * 16 + 4 * kq, false, av1, bv1);
+    load((sl + 1) * 16 + 4 * kq, false, av1, bv1);
     fma(av0, bv0);
     fma(av1, bv1);
   }
-  if (sl < nfull) {  // one full slab left
+  if (sl < end) {  // one full slab left
     double av[AT][4], bv[NT][4];
     load(sl * 16 + 4 * kq, false, av, bv);
     fma(av, bv);
   }
-  if (D % 16 != 0 && first == nfull % gx) {  // the partial last slab
+  if (D % 16 != 0 && first == gx - 1) {  // the partial last slab
     double av[AT][4], bv[NT][4];
     load(nfull * 16 + 4 * kq, true, av, bv);
     fma(av, bv);
@@ -167,71 +169,95 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(const double* __restri
   }
 }
 
-// B = beta*B + alpha*A*G.  Block: 4 waves, 64 rows (wave w: rows r0+16w..+15),
-// all n output columns (NT tiles of 16).  Contraction over the m columns of A
-// in steps of 4: A fragment lane l -> A[r0 + l%16, k + l/16] (16 consecutive
-// rows of one column), G fragment lane l -> G(k + l/16, 16t + l%16), element
-// (k, j) at G[k*gsk + j*gsj] (row-major G, gsj = 1, gives the 16 lanes of a
-// k-slot one 128-byte line).  Four steps' loads are issued before their
-// MFMAs.  Lanes past D or n read a clamped row or column (their results are
-// not stored); only the contraction slots past m in the last steps are zeroed.
-template <int NT>
+// B = beta*B + alpha*A*G.  Block: 4 waves; a wave takes 16*RT rows in RT tiles and
+// all n output columns (NT tiles of 16).  Lane l holds rows RT*(l%16) .. +RT-1 of its
+// wave (tile t the rows RT*i + t), so that one load of 8*RT bytes per lane serves RT
+// tiles and a fragment of G as many.  Contraction over the m columns of A in steps
+// of 4: column k + l/16 of A, G(k + l/16, 16t + l%16), element (k, j) at
+// G[k*gsk + j*gsj] (row-major G, gsj = 1, gives the 16 lanes of a k-slot one 128-byte
+// line).  Four steps' loads are issued before their MFMAs.  Lanes past D or n read
+// a clamped row or column (their results are not stored); only the contraction
+// slots past m in the last steps are zeroed.  RT = 2: 614 MB, 8 columns, in 122 us
+// (5.0 TB/s); one row per lane 151, four 121 but slower for 16 columns.
+template <int NT, int RT>
 __global__ __launch_bounds__(256) void update_kernel(const double* __restrict__ A, int64_t lda,
                                                      int m, const double* __restrict__ G,
                                                      int64_t gsk, int64_t gsj,
                                                      double* __restrict__ B, int64_t ldb, int n,
                                                      int64_t D, double alpha, double beta) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t r0 = (int64_t)blockIdx.x * 64 + w * 16;
   const int li = lane & 15, kq = lane >> 4;
-  const int64_t ra = r0 + li;
-  const double* pa = A + (ra < D ? ra : D - 1);
+  const int64_t r0 = ((int64_t)blockIdx.x * 64 + w * 16) * RT;
+  if (r0 >= D) return;
+  const int64_t ra = r0 + RT * li;
+  const bool tail = r0 + 16 * RT > D;  // (uniform)
+  typedef double vt __attribute__((ext_vector_type(RT)));
+  typedef double ut __attribute__((ext_vector_type(RT), aligned(8)));
+  auto load = [&](int64_t col) {
+    if (!tail) return (vt) * reinterpret_cast<const ut*>(A + ra + col * lda);
+    vt v;
+#pragma unroll
+    for (int q = 0; q < RT; ++q) v[q] = A[(ra + q < D ? ra + q : D - 1) + col * lda];
+    return v;
+  };
   const double* pg[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int j = t * 16 + li;
     pg[t] = G + (int64_t)(j < n ? j : n - 1) * gsj;
   }
-  d4 acc[NT];
+  d4 acc[RT][NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = (d4){0.0, 0.0, 0.0, 0.0};
+  for (int q = 0; q < RT; ++q)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[q][t] = (d4){0.0, 0.0, 0.0, 0.0};
   constexpr int U = 4;  // steps of 4 columns whose loads travel together
   int k = 0;
   for (; k + 4 * U <= m; k += 4 * U) {
-    double a[U], g[U][NT];
+    vt a[U];
+    double g[U][NT];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int ka = k + 4 * u + kq;
-      a[u] = pa[(int64_t)ka * lda];
+      a[u] = load(ka);
 #pragma unroll
       for (int t = 0; t < NT; ++t) g[u][t] = pg[t][ka * gsk];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = mfma16x16x4(a[u], g[u][t], acc[t]);
+      for (int q = 0; q < RT; ++q)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[q][t] = mfma16x16x4(a[u][q], g[u][t], acc[q][t]);
   }
   for (; k < m; k += 4) {
     const int ka = k + kq;
     const bool kok = ka < m;
     const int kc = kok ? ka : m - 1;
-    const double a = kok ? pa[(int64_t)kc * lda] : 0.0;
+    vt a = load(kc);
+    if (!kok) a = (vt)0.0;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = mfma16x16x4(a, pg[t][kc * gsk], acc[t]);
+    for (int t = 0; t < NT; ++t) {
+      const double g = pg[t][kc * gsk];
+#pragma unroll
+      for (int q = 0; q < RT; ++q) acc[q][t] = mfma16x16x4(a[q], g, acc[q][t]);
+    }
   }
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int j = t * 16 + li;
     if (j >= n) continue;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int64_t r = r0 + kq + 4 * v;
-      if (r < D) {
-        double* pb = B + r + (int64_t)j * ldb;
-        const double old = (beta == 0.0) ? 0.0 : beta * *pb;
-        *pb = old + alpha * acc[t][v];
+    for (int q = 0; q < RT; ++q)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t r = r0 + RT * (kq + 4 * v) + q;  // row kq + 4v of tile q
+        if (r < D) {
+          double* pb = B + r + (int64_t)j * ldb;
+          const double old = (beta == 0.0) ? 0.0 : beta * *pb;
+          *pb = old + alpha * acc[q][t][v];
+        }
       }
-    }
   }
 }
 
@@ -302,9 +328,8 @@ __device__ __forceinline__ void sum_partials(const double* __restrict__ part, in
 // One pass of Cholesky-QR in one block: G = W^T W from the Gram partials (nrb > 0) or
 // already summed in `part`, its factor R (G = R^T R) to Rout, R^-1 to Ri (both n x n,
 // column-major, upper).  With Rin (the second pass) Rout gets R * Rin.  A pivot that
-// is not positive and finite sets *fail (and *fail_host), and so does a set *prev;
-// every product is rounded (no fused multiply-add), so that the pivot of a repeated
-// column cancels to zero.
+// is not above its rounding, or not finite, sets *fail (and *fail_host), and so does a
+// set *prev; products are rounded (no fused multiply-add), as on a host.
 __global__ __launch_bounds__(1024) void chol_kernel(const double* __restrict__ part, int nrb, int n,
                                                     const double* __restrict__ Rin,
                                                     double* Rout, double* __restrict__ Ri,
@@ -313,7 +338,7 @@ __global__ __launch_bounds__(1024) void chol_kernel(const double* __restrict__ p
 #pragma clang fp contract(off)
   extern __shared__ double chol_lds[];
   double* G = chol_lds;             // G, then R (row j from column j on)
-  double* I = chol_lds + n * n;     // partial sums, then the inverse
+  double* I = chol_lds + n * n;     // partial sums, the columns' squared norms, the inverse
   const int t = threadIdx.x, nn = n * n;
   auto end = [&](int v) {
     if (t != 0) return;
@@ -327,11 +352,15 @@ __global__ __launch_bounds__(1024) void chol_kernel(const double* __restrict__ p
     for (int i = t; i < nn; i += 1024) G[i] = part[i];
   }
   __syncthreads();
+  if (t < n) I[t] = G[t * n + t];
+  __syncthreads();
   const int nt = n <= 16 ? 64 : 1024;  // (one wave: its barriers cost nothing)
   if (t >= nt) return;
   for (int j = 0; j < n; ++j) {
     const double d = G[j * n + j];
-    if (!(d > 0.0) || d > 1.7976931348623157e308) return end(1);  // (uniform)
+    // (a repeated column leaves up to four roundings of its norm, of either sign)
+    if (!(d > 4.0 * 2.220446049250313e-16 * I[j]) || d > 1.7976931348623157e308)
+      return end(1);  // (uniform)
     const double r = sqrt(d);
     __syncthreads();
     if (t == 0) G[j * n + j] = r;
@@ -420,10 +449,11 @@ static int gram_partials(pf_handle* h, const double* A, int64_t lda, int m, cons
                          int64_t ldb, int n, int64_t D, hipStream_t st) {
   const int nrb = (int)std::min<int64_t>(m <= 16 ? kGramRowBlocks1 : kGramRowBlocks, (D + 15) / 16);
   double* part = reinterpret_cast<double*>(h->partials.get((size_t)nrb * m * n * sizeof(double)));
-  // two A tiles per wave once A is wider than one block's 64 columns
-  const int AT = m > 64 ? 2 : 1;
-  dim3 grid(nrb, (m + 64 * AT - 1) / (64 * AT)), block(256);
+  // Two A tiles per wave where a wide B is loaded for each of them; with one tile of
+  // B, 416 columns take 136 us with one A tile per wave and 145 with two.
   const int NT = (n + 15) / 16;
+  const int AT = m > 64 && NT > 1 ? 2 : 1;
+  dim3 grid(nrb, (m + 64 * AT - 1) / (64 * AT)), block(256);
 #define PF_GRAM(...) \
   hipLaunchKernelGGL((gram_kernel<__VA_ARGS__>), grid, block, 0, st, A, lda, m, B, ldb, n, D, part)
   if (m <= 16) {
@@ -435,7 +465,6 @@ static int gram_partials(pf_handle* h, const double* A, int64_t lda, int m, cons
     }
   } else if (AT == 2) {
     switch (NT) {
-      case 1: PF_GRAM(1, 2); break;
       case 2: PF_GRAM(2, 2); break;
       case 3: PF_GRAM(3, 2); break;
       default: PF_GRAM(4, 2); break;
@@ -472,10 +501,11 @@ void update(const double* A, int64_t lda, int m, const double* G, int64_t gsk, i
   PF_REQUIRE(m >= 1 && n >= 1 && n <= kMaxN, "update: 1 <= n <= 64, m >= 1");
   PF_REQUIRE(D >= 1 && lda >= D && ldb >= D, "update: bad leading dimensions");
   PF_REQUIRE((gsk == 1 && gsj >= m) || (gsj == 1 && gsk >= n), "update: bad G layout");
-  dim3 grid((unsigned)((D + 63) / 64)), block(256);
+  constexpr int RT = 2;
+  dim3 grid((unsigned)((D + 64 * RT - 1) / (64 * RT))), block(256);
   const int NT = (n + 15) / 16;
 #define PF_UPDATE(NTV)                                                                         \
-  hipLaunchKernelGGL(update_kernel<NTV>, grid, block, 0, st, A, lda, m, G, gsk, gsj, B, ldb, n, \
+  hipLaunchKernelGGL((update_kernel<NTV, RT>), grid, block, 0, st, A, lda, m, G, gsk, gsj, B, ldb, n, \
                      D, alpha, beta)
   switch (NT) {
     case 1: PF_UPDATE(1); break;

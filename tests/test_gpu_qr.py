@@ -55,3 +55,21 @@ def test_lanczos_ortho_matches_numpy(dev, s, D):
                                b if prev else None, Wd)
         assert np.max(np.abs(got - a)) < 1e-14
         assert np.max(np.abs(dev.to_host(Wd) - (W - V @ a - (Vp @ b.T if prev else 0.0)))) < 1e-14
+
+
+@pytest.mark.parametrize("D", [1, 15, 17, 31, 127, 129, 4097])
+def test_gram_and_update_edges(dev, D):
+    """Rows at the edges of slabs, row pairs and row ranges; odd leading dimensions."""
+    from polfed_amd import blockops as bo
+    rng = np.random.default_rng(D)
+    for m, n in ((1, 1), (16, 8), (17, 1), (70, 17), (130, 64), (65, 33)):
+        A, B, G = rng.standard_normal((D, m)), rng.standard_normal((D, n)), rng.standard_normal((m, n))
+        pad = torch.full((m, D + 3), np.nan, dtype=torch.float64, device=dev.torch_device)
+        pad[:, :D] = dev.to_device(A)
+        out = torch.full((n, D + 1), 7.0, dtype=torch.float64, device=dev.torch_device)
+        out[:, :D] = dev.to_device(B)
+        got = dev.to_host(bo.gram(dev, pad[:, :D], out[:, :D]))
+        assert np.max(np.abs(got - A.T @ B)) < 1e-13 * max(D, 10)
+        bo.update(dev, pad[:, :D], dev.to_device(G), out[:, :D], alpha=-0.5, beta=2.0)
+        assert np.max(np.abs(dev.to_host(out[:, :D]) - (2.0 * B - 0.5 * A @ G))) < 1e-13 * max(m, 10)
+        assert (out[:, D:] == 7.0).all()
