@@ -251,7 +251,7 @@ TeamTables* team_build(const ChainParams& ref, const uint32_t* C, const uint32_t
 void team_destroy(TeamTables* t);
 int team_plan(const pf_op* op, int dtype, int polytype, int order, const double* X, int64_t ldx,
               const double* Y, int64_t ldy, int ncols);
-int team_best(const pf_op* op, int dtype, int ncols, double* us);
+int team_best(const pf_op* op, int dtype, int ncols, double* us, bool kpm = false);
 size_t team_work_bytes(const pf_op* op, int dtype, int order, int ncols, int T);
 void team_filter(pf_op* op, int dtype, int polytype, const double* coeffs, int order,
                  const double* X, int64_t ldx, double* Y, int64_t ldy, int ncols, int T,

@@ -158,8 +158,7 @@ __device__ __forceinline__ bool team_wait(TeamCtl* c, TeamPlace& me) {
   });
 }
 
-constexpr int kTeamThreads = 1024;
-constexpr int kTeamWaves = kTeamThreads / 64;
+constexpr int kTeamWaves = 16;  // most waves of a block
 
 // A value that is the same in all lanes, as a scalar.
 __device__ __forceinline__ uint32_t uni(uint32_t v) {

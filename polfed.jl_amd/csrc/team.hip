@@ -31,6 +31,8 @@
 //   L=14 FP64  1 column     4.8 -> 1.6      L=17 FP64  5 columns   5.3 -> 2.3
 //   L=20 FP64  8 columns   15.8 -> 6.7      L=20 FP32  8 columns  10.6 -> 5.4
 //   L=22 FP32 16 columns   57.0 -> 44.3     L=22 FP64 16 columns 124.5 -> 107 (streamed)
+//   J1-J2 FP64 8 columns: L=18 8.6 -> 5.9, L=20 26.2 -> 14.2; FP32: L=20 15.4 -> 9.6,
+//   L=21 28.5 -> 19.3
 
 #include <algorithm>
 #include <cstring>
@@ -42,6 +44,15 @@
 
 namespace pf {
 
+
+// Waves of a block: 16 with 128 registers, or eight with 256 where the resident FP64
+// forms spill otherwise (us a step, 16 and 8 waves: J1-J2 FP64 at L = 16 4.3 and
+// 3.0, L = 18 8.6 and 5.9, L = 20 30.0 and 14.3; XXZ FP64 at L = 21 17.2 and 14.8; but
+// XXZ FP64 at L = 20 6.8 and 8.4, J1-J2 FP32 at L = 20 9.6 and 12.7, and every
+// streamed column slower with eight).
+constexpr int team_waves(size_t elem, int NC, int R) {
+  return elem == 8 && ((NC == 6 && R > 0) || (NC == 2 && R == 14)) ? 8 : 16;
+}
 
 // kGrp consecutive rows of one segment, two per lane.
 constexpr uint32_t kGrp = 128;
@@ -349,18 +360,19 @@ struct TeamDots {
   }
 };
 // The block's sums of step j (all waves parked): written by two threads of wave 1.
+template <int W>
 __device__ __forceinline__ void team_dots_out(const TeamArgs& A, const TeamShared& sh, int j,
                                               int col, uint32_t idx) {
   if (threadIdx.x >= 64u && threadIdx.x < 66u) {
     const uint32_t w = threadIdx.x - 64u;
     double t = 0.0;
-    for (int i = 0; i < kTeamWaves; ++i) t += sh.red[2 * i + w];
+    for (int i = 0; i < W; ++i) t += sh.red[2 * i + w];
     A.dots[((int64_t)(2 * (j - 1) + (int)w) * A.ncols + col) * kTeamUnits + idx] = t;
   }
 }
 
 // The streaming form of one column (any team size, any D).
-template <typename T, int NQ, int NC, bool UNI, bool KPM>
+template <typename T, int NQ, int NC, bool UNI, bool KPM, int W>
 __device__ bool stream_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me, int col,
                               char* slot) {
   constexpr uint32_t sz = sizeof(T);
@@ -448,13 +460,13 @@ __device__ bool stream_column(const TeamArgs& A, TeamShared& sh, TeamPlace& me, 
       dots = TeamDots{};
     }
     if (j < steps && !team_step_end(A.ctl, sh, me, false, [&] {
-          if (KPM && !first) team_dots_out(A, sh, j, col, me.idx);
+          if (KPM && !first) team_dots_out<W>(A, sh, j, col, me.idx);
         }))
       return false;
   }
   if constexpr (KPM) {
     __syncthreads();
-    team_dots_out(A, sh, steps, col, me.idx);
+    team_dots_out<W>(A, sh, steps, col, me.idx);
   }
   return true;
 }
@@ -510,7 +522,8 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
                                                 int col, char* slot) {
   constexpr uint32_t sz = sizeof(T);
   typedef pair_t<T> pt;
-  constexpr bool kDiagReg = R * sizeof(T) <= 56;
+  constexpr int W = team_waves(sizeof(T), NC, R);
+  constexpr bool kDiagReg = R * W * sizeof(T) <= 56 * 16;
   constexpr int RN = rec_remote(NC);
   constexpr int LW = lrec_words(NC);
   const uint32_t lane = threadIdx.x & 63u;
@@ -523,10 +536,10 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
   double* Y = A.Y + (int64_t)col * A.ldy;
   const int mine = ge - ga - wave;  // groups r with 16 r < mine
   int left = mine;
-  auto have = [&](int r) { return r * kTeamWaves < left; };  // uniform
+  auto have = [&](int r) { return r * W < left; };  // uniform
   const uint32_t recs =
       A.tab_lds + ((uint32_t)wave * LW + (lane < (uint32_t)LW ? lane : LW - 1u)) * 4u;
-  auto rec_at = [&](int r) { return LRec{lread<uint32_t>(recs + (uint32_t)(r * kTeamWaves * LW * 4))}; };
+  auto rec_at = [&](int r) { return LRec{lread<uint32_t>(recs + (uint32_t)(r * W * LW * 4))}; };
   // the lane (the last pair's for lanes past the end), and whether it is one
   auto last_of = [&](const LRec& c) { return ((c[kRecCnt] & 0xFFu) - 1u) >> 1; };
   const uint32_t spare = A.rows_lds - 4u * sz;  // takes the writes of lanes without a row
@@ -570,7 +583,7 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
               lwrite<pt>(at, p[r]);
               p[r] = j == 1 ? (pt)(T)0 : t;  // (LDS is another column's then)
             }
-          if (KPM && j > 1) team_dots_out(A, sh, j - 1, col, me.idx);
+          if (KPM && j > 1) team_dots_out<W>(A, sh, j - 1, col, me.idx);
         }))
       return false;
     const __amdgpu_buffer_rsrc_t t = in;
@@ -683,7 +696,7 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
   }
   if constexpr (KPM) {
     __syncthreads();
-    team_dots_out(A, sh, A.order, col, me.idx);
+    team_dots_out<W>(A, sh, A.order, col, me.idx);
   }
   return true;
 }
@@ -691,7 +704,9 @@ __device__ __forceinline__ bool resident_column(const TeamArgs& A, TeamShared& s
 // R = 0: the streaming form only.  Dynamic LDS: class tables (at offset 0, so
 // that offsets need no base), then the form's own area, then TeamShared.
 template <typename T, int NQ, int NC, bool UNI, bool KPM, int R>
-__global__ __launch_bounds__(kTeamThreads) void chain_team_kernel(const TeamArgs A) {
+__global__ __launch_bounds__(64 * team_waves(sizeof(T), NC, R)) void
+chain_team_kernel(const TeamArgs A) {
+  constexpr int W = team_waves(sizeof(T), NC, R);
   TeamShared& sh = *reinterpret_cast<TeamShared*>(team_lds + A.rows_lds);
   // (team_enter in line: as a call, even inlined, the R = 4 form spills 34 registers
   // instead of 18 and a step at L = 20 takes 4 % longer)
@@ -708,7 +723,7 @@ __global__ __launch_bounds__(kTeamThreads) void chain_team_kernel(const TeamArgs
       }
     }
   }
-  for (uint32_t t = threadIdx.x * 8u; t < A.tab_lds; t += kTeamThreads * 8u)
+  for (uint32_t t = threadIdx.x * 8u; t < A.tab_lds; t += W * 64u * 8u)
     lwrite<uint64_t>(t, A.tab[t / 8u]);
   __syncthreads();
   if (!uni(sh.ok)) return;
@@ -725,10 +740,10 @@ __global__ __launch_bounds__(kTeamThreads) void chain_team_kernel(const TeamArgs
       const uint32_t* rec = A.rec + (int64_t)ga * rec_words(NC);
       // the block's first segment starts at element 4 of the rows
       const uint32_t base = ga < ge ? rows + (4u - rec[3]) * (uint32_t)sizeof(T) : 0u;
-      for (int t = threadIdx.x; t < (ge - ga) * LW; t += kTeamThreads)
+      for (int t = threadIdx.x; t < (ge - ga) * LW; t += W * 64)
         lwrite<uint32_t>(A.tab_lds + (uint32_t)t * 4u,
                          lrec_word<T, NC>(rec + (t / LW) * rec_words(NC), t % LW, base, A.elems));
-      for (uint32_t t = rows + threadIdx.x * 4u; t < A.rows_lds; t += kTeamThreads * 4u)
+      for (uint32_t t = rows + threadIdx.x * 4u; t < A.rows_lds; t += W * 64u * 4u)
         lwrite<uint32_t>(t, 0u);
     }
   }
@@ -747,9 +762,9 @@ __global__ __launch_bounds__(kTeamThreads) void chain_team_kernel(const TeamArgs
       ok = resident_column<T, NQ, NC, UNI, KPM, R>(A, sh, me, (int)col, work);
     } else if constexpr (R > 0) {
       ok = me.n == (uint32_t)A.T ? resident_column<T, NQ, NC, UNI, KPM, R>(A, sh, me, (int)col, work)
-                                 : stream_column<T, NQ, NC, UNI, KPM>(A, sh, me, (int)col, work);
+                                 : stream_column<T, NQ, NC, UNI, KPM, W>(A, sh, me, (int)col, work);
     } else {
-      ok = stream_column<T, NQ, NC, UNI, KPM>(A, sh, me, (int)col, work);
+      ok = stream_column<T, NQ, NC, UNI, KPM, W>(A, sh, me, (int)col, work);
     }
     if (!ok) return;
     if (threadIdx.x == 0 && me.idx == 0) (void)team_add(&A.ctl->done, 1u);
@@ -1058,7 +1073,7 @@ TeamTables* team_build(const ChainParams& ref, const uint32_t* C, const uint32_t
       }
       prev = sgrp[sg];
     }
-    if (T->maxgrp[lt] > 13 * kTeamWaves) continue;  // never resident
+    if (T->maxgrp[lt] > 13 * 16) continue;  // never resident
     // records; a target in the own block is given by its zero slot in LDS
     std::vector<uint32_t>& rc = rec[lt];
     rc.assign((size_t)T->ngrp * RW + 16, 0u);
@@ -1191,33 +1206,36 @@ static size_t team_resident_lds(const TeamTables* t, int lt, size_t sz) {
   return (team_table_bytes(t) + (size_t)t->maxgrp[lt] * lrec_words(t->NC) * 4 + 32 +
           ((size_t)t->maxel[lt] + 8) * sz + 31) & ~(size_t)31;
 }
-static size_t team_stream_lds(const TeamTables* t, size_t sz) {
-  return team_table_bytes(t) + ((size_t)kTeamWaves * t->maxseg + 8) * sz;
+static size_t team_stream_lds(const TeamTables* t, size_t sz, int R) {
+  return team_table_bytes(t) + ((size_t)team_waves(sz, t->NC, R) * t->maxseg + 8) * sz;
 }
 
 // Groups a wave holds in the resident form with 1 << lt blocks per column (the
-// kernel instance: 1, 2, 4, 7, 13), or 0 when the column does not fit.
-static int team_resident(const TeamTables* t, int dtype, int lt) {
+// kernel instance: 1, 2, 4, 7, 8, 13, 14), or 0 when the column does not fit.
+static int team_resident(const TeamTables* t, int dtype, int lt, bool kpm) {
   const size_t sz = dtype == PF_F64 ? 8 : 4;
   if (!t->rec[lt] || team_resident_lds(t, lt, sz) > kTeamLds) return 0;
-  const int need = (t->maxgrp[lt] + kTeamWaves - 1) / kTeamWaves;
-  const int most = dtype == PF_F64 ? (t->NQ == 3 ? 7 : 4) : (t->NQ == 3 ? 13 : 7);
-  for (const int r : {1, 2, 4, 7, 13})
-    if (need <= r && r <= most) return r;
+  const bool f64 = dtype == PF_F64;
+  for (const int r : {1, 2, 4, 7, 8, 13, 14}) {
+    const bool made = r <= 4 || (f64 ? r == (t->NC == 6 ? 8 : kpm ? 7 : 14)
+                                     : r == 7 || (r == 13 && t->NC == 2));
+    if (made && t->maxgrp[lt] <= r * team_waves(sz, t->NC, r)) return r;
+  }
   return 0;
 }
 
 // Time of one step on ncols columns with 1 << lt blocks per column, in us
-// (fitted to measurements on MI355X: one 128-row group per wave is 0.6 to 1.4 us
+// (fitted to measurements on MI355X: 16 128-row groups of a block are 1.0 to 3.8 us
 // in the resident form, the rest is the barrier; a streamed row is 0.05 to 0.12
 // ns).  Columns beyond 8 x 32 / T run in further rounds.
-static double team_step_us(const TeamTables* t, int dtype, int ncols, int lt) {
+static double team_step_us(const TeamTables* t, int dtype, int ncols, int lt, bool kpm) {
   const int T = 1 << lt;
   const int rounds = (ncols + 8 * (32 / T) - 1) / (8 * (32 / T));
   const bool f64 = dtype == PF_F64;
   double us = T == 32 ? 2.0 : T == 16 ? 1.6 : T == 1 ? 1.1 : 1.4;
-  if (team_resident(t, dtype, lt))
-    us += (double)t->maxgrp[lt] / kTeamWaves * (t->NQ == 3 ? (f64 ? 1.35 : 1.0) : (f64 ? 3.2 : 2.6));
+  if (const int R = team_resident(t, dtype, lt, kpm))
+    us += (double)t->maxgrp[lt] / 16 *
+          (t->NQ == 3 ? (f64 ? (R > 4 ? 1.9 : kpm ? 1.65 : 1.35) : 1.0) : (f64 ? 3.8 : 2.6));
   else
     us += (double)t->elems / T * (t->NQ == 3 ? (f64 ? 0.0021 : 0.0018) : (f64 ? 0.0042 : 0.0038));
   return rounds * us;
@@ -1235,7 +1253,7 @@ static double per_step_us(const pf_op* op, int dtype, int ncols) {
 int team_kpm_steps(int dtype, int N);
 
 // Blocks per column of the fastest team form, and its time.
-int team_best(const pf_op* op, int dtype, int ncols, double* us) {
+int team_best(const pf_op* op, int dtype, int ncols, double* us, bool kpm) {
   const TeamTables* t = op->team;
   int best = 0;
   *us = 1e300;
@@ -1252,7 +1270,7 @@ int team_best(const pf_op* op, int dtype, int ncols, double* us) {
   if (!t) return best;
   for (int lt = 0; lt < 6; ++lt) {
     if ((t->NC == 0) != (lt == 0)) continue;
-    const double x = team_step_us(t, dtype, ncols, lt);
+    const double x = team_step_us(t, dtype, ncols, lt, kpm);
     if (x < *us) {
       *us = x;
       best = 1 << lt;
@@ -1266,7 +1284,7 @@ constexpr int kTeamMinOrder = 8;
 
 // Blocks per column for `order` steps on ncols columns, or 0.  `gain`: the steps
 // that the per-step launches take for one of these.
-static int team_choose(const pf_op* op, int dtype, int order, int ncols, int gain) {
+static int team_choose(const pf_op* op, int dtype, int order, int ncols, int gain, bool kpm) {
   const TeamTables* t = op->team;
   const TuneCfg& f = op->force;
   const bool qsun = op->kind == kQsun && qsun_team_ok(op);
@@ -1278,11 +1296,12 @@ static int team_choose(const pf_op* op, int dtype, int order, int ncols, int gai
   if (order < kTeamMinOrder) return 0;
   // measured by the autotuner, else by the rule (by chunks of columns there)
   const auto it = op->tuned.find({dtype, ncols});
-  if (it != op->tuned.end() && (it->second.team > 0 || (it->second.team == 0 && gain == 1)))
-    return it->second.team;
+  const int tuned = it == op->tuned.end() ? -1 : it->second.team;
+  if (tuned > 0 && !kpm) return tuned;  // (the moments have their own best size)
+  if (tuned == 0 && gain == 1) return 0;
   double us;
-  const int T = team_best(op, dtype, ncols, &us);
-  return us < 0.95 * gain * per_step_us(op, dtype, ncols) ? T : 0;
+  const int T = team_best(op, dtype, ncols, &us, kpm);
+  return tuned > 0 || us < 0.95 * gain * per_step_us(op, dtype, ncols) ? T : 0;
 }
 
 int team_plan(const pf_op* op, int dtype, int polytype, int order, const double* X, int64_t ldx,
@@ -1292,7 +1311,7 @@ int team_plan(const pf_op* op, int dtype, int polytype, int order, const double*
   const double* xe = X + (ncols - 1) * ldx + op->D;
   const double* ye = Y + (ncols - 1) * ldy + op->D;
   if (X < ye && Y < xe && !(X == Y && ldx == ldy)) return 0;
-  return team_choose(op, dtype, order, ncols, 1);
+  return team_choose(op, dtype, order, ncols, 1, false);
 }
 
 // FP64 moments take half the steps here (TeamDots), so the team wins far above the
@@ -1301,7 +1320,8 @@ int team_plan(const pf_op* op, int dtype, int polytype, int order, const double*
 // L = 20 8.0 -> 5.3 ms, L = 18 2.9 -> 1.5 ms (team of 8).
 int team_kpm_plan(const pf_op* op, int dtype, int N, int ncols) {
   if (!op->team) return 0;
-  return team_choose(op, dtype, team_kpm_steps(dtype, N), ncols, dtype == PF_F64 ? 2 : 1);
+  return team_choose(op, dtype, team_kpm_steps(dtype, N), ncols, dtype == PF_F64 ? 2 : 1,
+                     true);
 }
 
 static size_t team_align(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -1330,7 +1350,7 @@ template <typename T, int NQ, int NC, bool UNI, bool KPM, int R>
 static void team_launch(const TeamArgs& A, int grid, size_t lds, hipStream_t st) {
   auto* k = chain_team_kernel<T, NQ, NC, UNI, KPM, R>;
   PF_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kTeamThreads), lds, st, A);
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(64 * team_waves(sizeof(T), NC, R)), lds, st, A);
   PF_HIP(hipGetLastError());
 }
 
@@ -1340,10 +1360,16 @@ static void team_launch_r(const TeamArgs& A, int R, int grid, size_t lds, hipStr
   if (R == 2) return team_launch<T, NQ, NC, UNI, KPM, 2>(A, grid, lds, st);
   if constexpr (NC > 0) {
     if (R == 4) return team_launch<T, NQ, NC, UNI, KPM, 4>(A, grid, lds, st);
-    if constexpr (NQ == 3 || sizeof(T) == 4)
+    if constexpr (sizeof(T) == 8) {
+      // (the recurrence of the moments holds no X, so 16 waves spill less: 32 columns at
+      // L = 20, blocks of 16 waves 3.71 ms, of eight 3.88)
+      constexpr int RM = NC == 6 ? 8 : KPM ? 7 : 14;
+      if (R == RM) return team_launch<T, NQ, NC, UNI, KPM, RM>(A, grid, lds, st);
+    } else {
       if (R == 7) return team_launch<T, NQ, NC, UNI, KPM, 7>(A, grid, lds, st);
-    if constexpr (NQ == 3 && sizeof(T) == 4)
-      if (R == 13) return team_launch<T, NQ, NC, UNI, KPM, 13>(A, grid, lds, st);
+      if constexpr (NC == 2)
+        if (R == 13) return team_launch<T, NQ, NC, UNI, KPM, 13>(A, grid, lds, st);
+    }
     if (R == 0) return team_launch<T, NQ, NC, UNI, KPM, 0>(A, grid, lds, st);
   }
   throw Error{PF_ERR_UNSUPPORTED, "team filter: no kernel for this plan"};
@@ -1376,7 +1402,7 @@ static void team_run(pf_op* op, int dtype, TeamArgs A, int T, void* work, size_t
   p += team_align(coef_bytes);
   int lt = 0;
   while ((1 << lt) < T) ++lt;
-  const int R = team_resident(t, dtype, lt);
+  const int R = team_resident(t, dtype, lt, kpm);
   const Affine af = op->affine(true);
   A.tab = t->tab[w];
   A.grp = t->grp;
@@ -1410,7 +1436,7 @@ static void team_run(pf_op* op, int dtype, TeamArgs A, int T, void* work, size_t
   const int grid = std::max(T, cus / nxcd * nxcd);
   A.expect = grid / nxcd;
   size_t lds = R ? team_resident_lds(t, lt, sz) : team_table_bytes(t);
-  if (t->NC > 0) lds = std::max(lds, team_stream_lds(t, sz));
+  if (t->NC > 0) lds = std::max(lds, team_stream_lds(t, sz, R));
   lds = (lds + 31) & ~(size_t)31;
   A.rows_lds = (uint32_t)lds;
   lds += sizeof(TeamShared);

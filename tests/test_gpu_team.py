@@ -31,6 +31,9 @@ CASES = [
     ("cut_ring_j1j2", 14, 7, 0.5, "periodic", 3, [1, 2, 32]),
     ("few_particles", 20, 4, 0.0, "periodic", 17, [1, 8, 32]),
     ("many_particles", 16, 12, 0.5, "open", 2, [2, 16]),
+    # the most groups per wave (blocks of eight waves in FP64), and too many
+    ("ring_xxz_full", 18, 9, 0.0, "periodic", 1, [2, 4, 8]),
+    ("ring_j1j2_full", 18, 9, 0.5, "periodic", 1, [4, 8, 16]),
 ]
 
 
